@@ -3,7 +3,7 @@
 island.hip is compiled once per (gene-block count, algorithm family) pair of the
 LDS-resident kernel and once per (row-tile count, algorithm family) pair of the
 wide kernel; each object holds one kernel that dispatches per task to an
-objective-specialised body.  The objects are linked with the host runtime into
+objective-specialised body.  objective.hip is compiled once per row-tile count.  The objects are linked with the host runtime into
 sg-emtf_amd/libemtf.so.
 """
 import os
@@ -26,6 +26,9 @@ VARIANTS = [(kb, al) for kb in (2, 4, 7, 8, 12, 13, 16) for al in (0, 2)]
 # wide kernel: (32-row tiles NT: dims <= 32 NT, rows in global memory; algorithm family)
 WIDE = [(nt, al) for nt in (2, 4, 5, 6, 7, 8) for al in (0, 2)]
 
+# objective / adjoint operator: 32-row tiles NT (dims <= 32 NT)
+OBJECTIVE = range(1, 9)
+
 
 def _run(cmd):
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -44,6 +47,8 @@ def build(verbose=False, jobs=None, out=None, extra=()):
     units += [([HIPCC] + COMMON + list(extra) + [f"-DEMTF_WIDE_NT={nt}", f"-DEMTF_ALGO={al}", "-c",
                                    "-o", os.path.join(OBJ, f"island_w{nt}_a{al}.o"), os.path.join(CSRC, "island.hip")])
               for nt, al in WIDE]
+    units += [([HIPCC] + COMMON + list(extra) + [f"-DEMTF_OBJ_NT={nt}", "-c", "-o", os.path.join(OBJ, f"objective_nt{nt}.o"),
+                                   os.path.join(CSRC, "objective.hip")]) for nt in OBJECTIVE]
     for name in ("emtf_host.cpp", "cvrp_host.cpp", "cvrp.hip", "export.hip"):
         units.append([HIPCC] + COMMON + ["-c", "-o", os.path.join(OBJ, name.split(".")[0] + ".o"), os.path.join(CSRC, name)])
     with ThreadPoolExecutor(jobs) as ex:
@@ -56,6 +61,7 @@ def build(verbose=False, jobs=None, out=None, extra=()):
             print(msg)
     objs = [os.path.join(OBJ, f"island_kb{kb}_a{al}.o") for kb, al in VARIANTS] + \
         [os.path.join(OBJ, f"island_w{nt}_a{al}.o") for nt, al in WIDE] + \
+        [os.path.join(OBJ, f"objective_nt{nt}.o") for nt in OBJECTIVE] + \
         [os.path.join(OBJ, n + ".o") for n in ("emtf_host", "cvrp_host", "cvrp", "export")]
     rc, msg = _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out + ".tmp"] + objs)
     if rc != 0:

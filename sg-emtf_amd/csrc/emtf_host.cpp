@@ -50,15 +50,16 @@ EMTF_DECL_WPAIR(2) EMTF_DECL_WPAIR(4) EMTF_DECL_WPAIR(5) EMTF_DECL_WPAIR(6) EMTF
     extern "C" int emtf_wideq_lds_floats_nt##nt##_a##al(int pop);
 #define EMTF_DECL_QPAIR(nt) EMTF_DECL_WIDEQ(nt, 0) EMTF_DECL_WIDEQ(nt, 2)
 EMTF_DECL_QPAIR(2) EMTF_DECL_QPAIR(4) EMTF_DECL_QPAIR(5) EMTF_DECL_QPAIR(6)
-#define EMTF_DECL_OBJ(kb)                                                                                   \
-    extern "C" int emtf_launch_objective_kb##kb(const emtf::ObjArgs* a, int adjoint, hipStream_t s);      \
+#define EMTF_DECL_POLISH(kb)                                                                                \
     extern "C" int emtf_polish_lds_floats_kb##kb(int pop, int waves, int cpe);                             \
     extern "C" int emtf_launch_polish_kb##kb(const emtf::EpochArgs* args, const int* order, int n, int lds_bytes, \
                                              hipStream_t stream);
-EMTF_DECL_OBJ(2) EMTF_DECL_OBJ(4) EMTF_DECL_OBJ(7) EMTF_DECL_OBJ(8) EMTF_DECL_OBJ(12) EMTF_DECL_OBJ(13) EMTF_DECL_OBJ(16)
-// forward objective for 128 < dim <= 32 NT (Q and points read from global memory)
-#define EMTF_DECL_OBJW(nt) extern "C" int emtf_launch_objective_nt##nt##_fwd(const emtf::ObjArgs* a, hipStream_t s);
-EMTF_DECL_OBJW(5) EMTF_DECL_OBJW(6) EMTF_DECL_OBJW(7) EMTF_DECL_OBJW(8)
+EMTF_DECL_POLISH(2) EMTF_DECL_POLISH(4) EMTF_DECL_POLISH(7) EMTF_DECL_POLISH(8) EMTF_DECL_POLISH(12)
+EMTF_DECL_POLISH(13) EMTF_DECL_POLISH(16)
+// objective / adjoint for dim <= 32 NT (adjoint: NT <= 4)
+#define EMTF_DECL_OBJN(nt) extern "C" int emtf_launch_objective_nt##nt(const emtf::ObjArgs* a, int adjoint, hipStream_t s);
+EMTF_DECL_OBJN(1) EMTF_DECL_OBJN(2) EMTF_DECL_OBJN(3) EMTF_DECL_OBJN(4)
+EMTF_DECL_OBJN(5) EMTF_DECL_OBJN(6) EMTF_DECL_OBJN(7) EMTF_DECL_OBJN(8)
 
 // the persistent schedule's kernel (LDS kernel builds) and its occupancy query
 #define EMTF_DECL_PERSIST(kb, al)                                                                           \
@@ -1393,25 +1394,10 @@ static int objective_call(int32_t func, int32_t dim, int32_t n, const float* x, 
     a.f = f;
     a.gx = gx;
     func_table(func, dim, a.tab);
-    int rc = -1;
-    if (dim > 128) {
-        switch (pick_nt(dim)) {
-        case 5: rc = emtf_launch_objective_nt5_fwd(&a, (hipStream_t)stream); break;
-        case 6: rc = emtf_launch_objective_nt6_fwd(&a, (hipStream_t)stream); break;
-        case 7: rc = emtf_launch_objective_nt7_fwd(&a, (hipStream_t)stream); break;
-        case 8: rc = emtf_launch_objective_nt8_fwd(&a, (hipStream_t)stream); break;
-        }
-    } else {
-        switch (pick_kb(dim)) {
-        case 2: rc = emtf_launch_objective_kb2(&a, adjoint, (hipStream_t)stream); break;
-        case 4: rc = emtf_launch_objective_kb4(&a, adjoint, (hipStream_t)stream); break;
-        case 7: rc = emtf_launch_objective_kb7(&a, adjoint, (hipStream_t)stream); break;
-        case 8: rc = emtf_launch_objective_kb8(&a, adjoint, (hipStream_t)stream); break;
-        case 12: rc = emtf_launch_objective_kb12(&a, adjoint, (hipStream_t)stream); break;
-        case 13: rc = emtf_launch_objective_kb13(&a, adjoint, (hipStream_t)stream); break;
-        case 16: rc = emtf_launch_objective_kb16(&a, adjoint, (hipStream_t)stream); break;
-        }
-    }
+    static const auto launchers = {emtf_launch_objective_nt1, emtf_launch_objective_nt2, emtf_launch_objective_nt3,
+                                   emtf_launch_objective_nt4, emtf_launch_objective_nt5, emtf_launch_objective_nt6,
+                                   emtf_launch_objective_nt7, emtf_launch_objective_nt8};
+    const int rc = launchers.begin()[(dim + 31) / 32 - 1](&a, adjoint, (hipStream_t)stream);
     if (rc != 0) return fail(EMTF_E_DEVICE, std::string("objective kernel launch: ") + hipGetErrorString((hipError_t)rc));
     return EMTF_OK;
 }

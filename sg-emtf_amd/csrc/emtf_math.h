@@ -320,4 +320,11 @@ struct FastMod {
     }
 };
 
+// LDS written by a wave and read by its other lanes: the wave's own order, no barrier.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace emtf

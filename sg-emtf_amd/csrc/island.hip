@@ -27,12 +27,11 @@
 // stride.  Slots past the task's dimension hold zeros, which makes every MFMA
 // step and every gene block unconditional: padded steps add +0 products.
 #include <hip/hip_runtime.h>
+#include "emtf_eval.h"
 #include "emtf_math.h"
 #include "emtf_types.h"
 
 namespace emtf {
-
-typedef float f16v __attribute__((ext_vector_type(16)));
 
 constexpr int kThreads = 256;
 
@@ -64,9 +63,6 @@ __host__ __device__ inline int lds_floats_kb(int pop, int kb) {
     const int RS = 8 * kb + 4, NT = (kb + 3) / 4, popP = (pop + 31) & ~31;
     return popP * RS + 32 * NT * RS + RS + 32 * NT + 4 * popP;
 }
-
-__device__ __forceinline__ float4 lds4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float f4(const float4& v, int e) { return e == 0 ? v.x : (e == 1 ? v.y : (e == 2 ? v.z : v.w)); }
 
 // v clamped to [lo, hi] (hi if v > hi, else lo if v < lo, else v: a NaN stays NaN), as
 // two selects.
@@ -126,412 +122,6 @@ __device__ __forceinline__ int pick_donor(const EpochArgs& a, int task, uint32_t
         else hi = mid;
     }
     return a.donors[k + (k >= lo ? 1 : 0)];
-}
-
-// ---------------------------------------------------------------------------
-// Objective of the lane's individual from its MFMA accumulators.
-// Lane (col, h) holds z_j for j = 32 jt + 8 (r >> 2) + 4 h + (r & 3); the two
-// halves accumulate the even / odd blocks of four rows in increasing j and
-// are combined once.
-// ZPAD: the caller's Q rows past D are zero, so z_j = +0 there; the objectives whose
-// term at z = +0 is +0 (whose sums it leaves as they are, bit for bit: they start at
-// +0 and never reach -0) and costs what any other row's does then add those rows
-// unmasked.  (Weierstrass keeps the mask: at z = 0 its term takes the small-|z| branch,
-// which would diverge from the other rows of the same slot.)
-// ---------------------------------------------------------------------------
-template <int FUNC>
-constexpr bool zero_term_at_zero() {
-    return FUNC == F_SPHERE || FUNC == F_ELLIPTIC || FUNC == F_ACKLEY || FUNC == F_RASTRIGIN ||
-           FUNC == F_GRIEWANK || FUNC == F_SCHWEFEL || FUNC == F_REF_RASTRIGIN;
-}
-
-// The objective's terms and final combination in split form, for the polish's line search
-// (terms of a row tile computed apart from the running sums): the same operations, in the
-// same order, as objective() below, which keeps them inline for the epoch kernels' code.
-//
-// Rosenbrock's term of row j (z = z_j, zn = z_{j+1}); it counts when row j + 1 exists.
-__device__ __forceinline__ float rosen_val(float z, float zn) {
-    const float zz = z * z;
-    const float a = zz - zn;
-    const float b = z - 1.0f;
-    float t1 = 100.0f * a;
-    t1 = t1 * a;
-    const float b2 = b * b;
-    return t1 + b2;
-}
-
-// The term values of row j of every textbook objective but Rosenbrock (v2: Ackley's
-// cosine term, Griewank's 2 sin^2); the Weierstrass term only for rows j < Dm (0 otherwise).
-template <int FUNC>
-__device__ __forceinline__ void row_vals(float z, int j, int Dm, const float* tab, float& v1, float& v2) {
-    static_assert(FUNC <= F_ELLIPTIC, "textbook objectives only");
-    if constexpr (FUNC == F_SPHERE) {
-        v1 = z * z;
-    } else if constexpr (FUNC == F_ELLIPTIC) {
-        const float zz = z * z;
-        v1 = tab[j] * zz;
-    } else if constexpr (FUNC == F_ACKLEY) {
-        v1 = z * z;
-        v2 = sinpi_sq(z);
-    } else if constexpr (FUNC == F_RASTRIGIN) {
-        const float zz = z * z;
-        const float s20 = 20.0f * sinpi_sq(z);
-        v1 = zz + s20;
-    } else if constexpr (FUNC == F_GRIEWANK) {
-        v1 = z * z;
-        v2 = 2.0f * sinpi_sq(z * tab[j]);
-    } else if constexpr (FUNC == F_WEIERSTRASS) {
-        v1 = 0.0f;
-        if (j < Dm) v1 = weier_term(z);
-    } else if constexpr (FUNC == F_SCHWEFEL) {
-        const float sq = sqrtf(__builtin_fabsf(z));
-        const float tv = sq * 0.159154937f;
-        v1 = z * sin2pi(tv);
-    }
-}
-
-// Adds one row's term values into the lane's sums (s2: Ackley's cosine sum, Griewank's
-// running 1 - prod cos) when the row counts.
-template <int FUNC>
-__device__ __forceinline__ void row_sum(float v1, float v2, bool in, float& s1, float& s2) {
-    if (!in) return;
-    s1 = s1 + v1;
-    if constexpr (FUNC == F_ACKLEY) {
-        s2 = s2 + v2;
-    } else if constexpr (FUNC == F_GRIEWANK) {
-        const float om = 1.0f - s2;
-        const float aq = v2 * om;
-        s2 = s2 + aq;
-    }
-}
-
-// The fitness from the two halves' sums (lane h holds its half's s1, s2; the other
-// half's come over the cross-half shuffle), textbook objectives.
-template <int FUNC>
-__device__ __forceinline__ float objective_tail(float s1, float s2, int D, const float* tab, int h) {
-    static_assert(FUNC <= F_ELLIPTIC, "textbook objectives only");
-    const float o1 = __shfl_xor(s1, 32);
-    const float S = s1 + o1;  // A + B (commutative)
-    const float Df = (float)D;
-    if constexpr (FUNC == F_ACKLEY) {
-        const float o2 = __shfl_xor(s2, 32);
-        const float C = s2 + o2;
-        const float q = S / Df;
-        const float r = sqrtf(q);
-        const float a = -0.2f * r;
-        const float t1 = -20.0f * expm1_f(a);
-        const float c2 = C / Df;
-        const float b = -2.0f * c2;
-        const float t2 = 2.71828175f * expm1_f(b);
-        return t1 - t2;
-    } else if constexpr (FUNC == F_GRIEWANK) {
-        const float o2 = __shfl_xor(s2, 32);
-        const float qA = h ? o2 : s2;
-        const float qB = h ? s2 : o2;
-        const float om = 1.0f - qA;
-        const float tq = qB * om;
-        const float Qv = qA + tq;
-        const float s4 = S / 4000.0f;
-        return s4 + Qv;
-    } else if constexpr (FUNC == F_SCHWEFEL) {
-        // the constant from the task table: 418.982887 (textbook) or 418.9829 (reference)
-        const float cd = tab[0] * Df;
-        return cd - S;
-    } else {
-        return S;
-    }
-}
-
-template <int NT, int FUNC, bool SKIP = false, bool ZPAD = false>
-__device__ __forceinline__ float objective(const f16v (&acc)[NT], int D, const float* tab, int h) {
-    // the row mask's bound: with ZPAD one no row reaches
-    const int Dm = (ZPAD && zero_term_at_zero<FUNC>()) ? 0x7FFFFFFF : D;
-    float s1 = 0.0f, s2 = (FUNC == F_REF_GRIEWANK) ? 1.0f : 0.0f;
-    if constexpr (FUNC == F_ROSENBROCK) {
-        float nb[NT][4];
-#pragma unroll
-        for (int jt = 0; jt < NT; ++jt)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) nb[jt][g] = __shfl_xor(acc[jt][4 * g], 32);
-#pragma unroll
-        for (int jt = 0; jt < NT; ++jt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int j = 32 * jt + 8 * (r >> 2) + 4 * h + (r & 3);
-                const int g = r >> 2;
-                float zn;
-                if ((r & 3) != 3) zn = acc[jt][r + 1];
-                else if (g < 3) zn = h ? nb[jt][g + 1] : nb[jt][g];
-                else zn = h ? ((jt + 1 < NT) ? nb[(jt + 1) % NT][0] : 0.0f) : nb[jt][g];
-                const float z = acc[jt][r];
-                const float zz = z * z;
-                const float a = zz - zn;
-                const float b = z - 1.0f;
-                float t1 = 100.0f * a;
-                t1 = t1 * a;
-                const float b2 = b * b;
-                const float v = t1 + b2;
-                if (j + 1 < D) s1 = s1 + v;
-            }
-    } else if constexpr (FUNC == F_WEIERSTRASS && SKIP && !ZPAD) {
-        // The wide kernels (SKIP, rows not zero-padded): four rows at a time, their terms
-        // by the branch-free path (independent chains the scheduler interleaves), the rare
-        // arguments redone by the full term, then the row sums in row order as below (s1 is
-        // never -0, so adding +0 for a masked row leaves it).  The LDS epoch kernel keeps
-        // one row at a time: there the interleaved chains take issue slots from the tasks
-        // that share the CU and the mixed epoch is slower.
-#pragma unroll
-        for (int jt = 0; jt < NT; ++jt)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                if (32 * jt + 8 * g >= D) continue;
-                float v[4];
-                bool rare = false;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float a = __builtin_fabsf(acc[jt][4 * g + e]);
-                    const bool lo = a >= 2.32830644e-10f, hi = a >= 8388608.0f;
-                    v[e] = weier_core(a, lo && !hi);
-                    rare = rare || (!lo && !hi && a != 0.0f);  // NaN or 0 < |z| < 2^-32
-                }
-                if (rare) {
-                    // one inlined copy of the full term: a rolled loop, the row picked by selects
-#pragma unroll 1
-                    for (int e = 0; e < 4; ++e) {
-                        float z = acc[jt][4 * g];
-                        z = e == 1 ? acc[jt][4 * g + 1] : z;
-                        z = e == 2 ? acc[jt][4 * g + 2] : z;
-                        z = e == 3 ? acc[jt][4 * g + 3] : z;
-                        const float a = __builtin_fabsf(z);
-                        if (z != z || (a > 0.0f && a < 2.32830644e-10f)) {
-                            const float r = weier_term(z);
-#pragma unroll
-                            for (int f = 0; f < 4; ++f) v[f] = e == f ? r : v[f];
-                        }
-                    }
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int j = 32 * jt + 8 * g + 4 * h + e;
-                    s1 = s1 + (j < Dm ? v[e] : 0.0f);
-                }
-            }
-    } else {
-        // SKIP: groups of eight rows past the dimension are skipped outright (a
-        // uniform branch) for the objectives with transcendental terms -- worth it
-        // where the row tiles are padded far past D (the wide kernel) or the terms are
-        // costly (Weierstrass, Schwefel in the LDS kernel); rows j >= D are masked in
-        // every case
-        constexpr bool skip = SKIP && FUNC != F_SPHERE && FUNC != F_ELLIPTIC;
-#pragma unroll
-        for (int jt = 0; jt < NT; ++jt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                if (skip && 32 * jt + 8 * (r >> 2) >= D) continue;
-                const int j = 32 * jt + 8 * (r >> 2) + 4 * h + (r & 3);
-                const float z = acc[jt][r];
-                if constexpr (FUNC == F_SPHERE) {
-                    const float v = z * z;
-                    if (j < Dm) s1 = s1 + v;
-                } else if constexpr (FUNC == F_ELLIPTIC) {
-                    const float zz = z * z;
-                    const float v = tab[j] * zz;
-                    if (j < Dm) s1 = s1 + v;
-                } else if constexpr (FUNC == F_ACKLEY) {
-                    const float v = z * z;
-                    const float sq = sinpi_sq(z);
-                    if (j < Dm) { s1 = s1 + v; s2 = s2 + sq; }
-                } else if constexpr (FUNC == F_RASTRIGIN) {
-                    const float zz = z * z;
-                    const float s20 = 20.0f * sinpi_sq(z);
-                    const float v = zz + s20;
-                    if (j < Dm) s1 = s1 + v;
-                } else if constexpr (FUNC == F_GRIEWANK) {
-                    const float v = z * z;
-                    const float a = 2.0f * sinpi_sq(z * tab[j]);
-                    if (j < Dm) {
-                        s1 = s1 + v;
-                        const float om = 1.0f - s2;
-                        const float aq = a * om;
-                        s2 = s2 + aq;
-                    }
-                } else if constexpr (FUNC == F_WEIERSTRASS) {
-                    if (j < Dm) s1 = s1 + weier_term(z);
-                } else if constexpr (FUNC == F_SCHWEFEL) {
-                    const float sq = sqrtf(__builtin_fabsf(z));
-                    const float tv = sq * 0.159154937f;
-                    const float v = z * sin2pi(tv);
-                    if (j < Dm) s1 = s1 + v;
-                } else if constexpr (FUNC == F_REF_ACKLEY) {
-                    // the reference's terms: z^2 and cospif(2 z)
-                    const float v = z * z;
-                    const float tz = 2.0f * z;
-                    const float c = cospi_f(tz);
-                    if (j < Dm) { s1 = s1 + v; s2 = s2 + c; }
-                } else if constexpr (FUNC == F_REF_RASTRIGIN) {
-                    // z^2 - 10 cospif(2 z) + 10
-                    const float zz = z * z;
-                    const float tz = 2.0f * z;
-                    const float c = cospi_f(tz);
-                    const float t = 10.0f * c;
-                    float v = zz - t;
-                    v = v + 10.0f;
-                    if (j < Dm) s1 = s1 + v;
-                } else if constexpr (FUNC == F_REF_GRIEWANK) {
-                    // z^2 and the factor cosf(z / sqrtf(j + 1)), cos q = 1 - 2 sin^2(q / 2)
-                    const float v = z * z;
-                    const float q = z / tab[j];
-                    const float tq = q * 0.159154937f;
-                    const float t = 2.0f * sinpi_sq(tq);
-                    const float c = 1.0f - t;
-                    if (j < Dm) { s1 = s1 + v; s2 = s2 * c; }
-                } else if constexpr (FUNC == F_REF_WEIERSTRASS) {
-                    if (j < Dm) s1 = s1 + weier_ref_term(z);
-                }
-            }
-    }
-    const float o1 = __shfl_xor(s1, 32);
-    const float S = s1 + o1;  // A + B (commutative)
-    const float Df = (float)D;
-    if constexpr (FUNC == F_ACKLEY) {
-        const float o2 = __shfl_xor(s2, 32);
-        const float C = s2 + o2;
-        const float q = S / Df;
-        const float r = sqrtf(q);
-        const float a = -0.2f * r;
-        const float t1 = -20.0f * expm1_f(a);
-        const float c2 = C / Df;
-        const float b = -2.0f * c2;
-        const float t2 = 2.71828175f * expm1_f(b);
-        return t1 - t2;
-    } else if constexpr (FUNC == F_GRIEWANK) {
-        const float o2 = __shfl_xor(s2, 32);
-        const float qA = h ? o2 : s2;
-        const float qB = h ? s2 : o2;
-        const float om = 1.0f - qA;
-        const float tq = qB * om;
-        const float Qv = qA + tq;
-        const float s4 = S / 4000.0f;
-        return s4 + Qv;
-    } else if constexpr (FUNC == F_SCHWEFEL) {
-        // the constant from the task table: 418.982887 (textbook) or 418.9829 (reference)
-        const float cd = tab[0] * Df;
-        return cd - S;
-    } else if constexpr (FUNC == F_REF_ACKLEY) {
-        // -20 expf(-0.2 sqrtf(S / D)) - expf(C / D) + 20 + E with the reference's double
-        // literals -0.2 and E = 2.718282 (SG-EMTF_DE.cu:913)
-        const float o2 = __shfl_xor(s2, 32);
-        const float C = s2 + o2;
-        const float q = S / Df;
-        const float r = sqrtf(q);
-        const float a = (float)(-0.2 * (double)r);
-        const float t1 = -20.0f * exp_f(a);
-        const float c2 = C / Df;
-        const float e2 = exp_f(c2);
-        float u = t1 - e2;
-        u = u + 20.0f;
-        return (float)((double)u + 2.718282);
-    } else if constexpr (FUNC == F_REF_GRIEWANK) {
-        // 1 + S / 4000 - prod (the halves' partial products multiplied once)
-        const float o2 = __shfl_xor(s2, 32);
-        const float P = s2 * o2;
-        const float s4 = S / 4000.0f;
-        const float u = 1.0f + s4;
-        return u - P;
-    } else if constexpr (FUNC == F_REF_WEIERSTRASS) {
-        // sum - D W with the reference's constant W in the task table
-        const float dw = Df * tab[0];
-        return S - dw;
-    } else {
-        return S;
-    }
-}
-
-// One 32-row tile (tile jt, accumulators acc) of the objective, in two parts: the row
-// terms (independent of every other tile; zn0: Rosenbrock's z of row 32 (jt + 1) for this
-// column, 0 past the last tile), then their sums onto the lane's running s1, s2 -- the
-// rows of tile jt in the order objective() adds them.
-template <int FUNC>
-__device__ __forceinline__ void tile_vals(const f16v& acc, int jt, int D, const float* tab, int h, float zn0,
-                                          float (&v1)[16], float (&v2)[16]) {
-    if constexpr (FUNC == F_ROSENBROCK) {
-        float nb[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) nb[g] = __shfl_xor(acc[4 * g], 32);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int g = r >> 2;
-            float zn;
-            if ((r & 3) != 3) zn = acc[r + 1];
-            else if (g < 3) zn = h ? nb[g + 1] : nb[g];
-            else zn = h ? zn0 : nb[g];
-            v1[r] = rosen_val(acc[r], zn);
-            v2[r] = 0.0f;
-        }
-    } else if constexpr (FUNC == F_WEIERSTRASS) {
-        // four rows at a time through the branch-free term (as in the wide kernels'
-        // objective), groups of eight rows past D skipped (a uniform branch); v1 = 0 for the
-        // masked rows as row_vals gives
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v1[4 * g + e] = 0.0f;
-                v2[4 * g + e] = 0.0f;
-            }
-            if (32 * jt + 8 * g >= D) continue;
-            float v[4];
-            bool rare = false;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float a = __builtin_fabsf(acc[4 * g + e]);
-                const bool lo = a >= 2.32830644e-10f, hi = a >= 8388608.0f;
-                v[e] = weier_core(a, lo && !hi);
-                rare = rare || (!lo && !hi && a != 0.0f);  // NaN or 0 < |z| < 2^-32
-            }
-            if (rare) {
-#pragma unroll 1
-                for (int e = 0; e < 4; ++e) {
-                    float z = acc[4 * g];
-                    z = e == 1 ? acc[4 * g + 1] : z;
-                    z = e == 2 ? acc[4 * g + 2] : z;
-                    z = e == 3 ? acc[4 * g + 3] : z;
-                    const float a = __builtin_fabsf(z);
-                    if (z != z || (a > 0.0f && a < 2.32830644e-10f)) {
-                        const float r = weier_term(z);
-#pragma unroll
-                        for (int f = 0; f < 4; ++f) v[f] = e == f ? r : v[f];
-                    }
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int j = 32 * jt + 8 * g + 4 * h + e;
-                v1[4 * g + e] = j < D ? v[e] : 0.0f;
-            }
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            v1[r] = 0.0f;
-            v2[r] = 0.0f;
-            row_vals<FUNC>(acc[r], 32 * jt + 8 * (r >> 2) + 4 * h + (r & 3), D, tab, v1[r], v2[r]);
-        }
-    }
-}
-
-template <int FUNC>
-__device__ __forceinline__ void tile_sums(const float (&v1)[16], const float (&v2)[16], int jt, int D, int h, float& s1,
-                                          float& s2) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int j = 32 * jt + 8 * (r >> 2) + 4 * h + (r & 3);
-        if constexpr (FUNC == F_ROSENBROCK) {
-            if (j + 1 < D) s1 = s1 + v1[r];
-        } else {
-            row_sum<FUNC>(v1[r], v2[r], j < D, s1, s2);
-        }
-    }
 }
 
 // z = Q (x - o) for the 32 individuals of a tile (x: the lane's parity half)
@@ -1086,138 +676,14 @@ __device__ __forceinline__ void transfer_in(const EpochArgs& a, const TaskDev& t
     __syncthreads();
 }
 
-// ---------------------------------------------------------------------------
-// Stand-alone objective and adjoint (emtf_objective_fwd / emtf_objective_adjoint).
-// A wave evaluates 32 points.  The forward pass is the engine's evaluator (bit
-// for bit).  The adjoint forms dz = df/dz per dimension in binary32 from z
-// staged in LDS, scales it by the upstream gradient, and contracts
-// gx = Q^T dz with a second run of v_mfma_f32_32x32x2_f32 (A = Q read
-// transposed from LDS, B = dz with one point per column).
-// ---------------------------------------------------------------------------
-template <int KB>
-struct ObjShape {
-    static constexpr int PB = (KB <= 8) ? 128 : 32;  // points per workgroup
-    static constexpr int ZS = 32 * Shape<KB>::NT + 1; // LDS stride of staged z rows
-};
-
-template <int KB>
-__host__ __device__ inline int obj_lds_floats() {
-    using S = Shape<KB>;
-    constexpr int PB = ObjShape<KB>::PB, ZS = ObjShape<KB>::ZS;
-    return 32 * S::NT * S::RS + S::RS + 32 * S::NT + 2 * PB * ZS;
-}
-
-// Per-point factors of d f / d z: Ackley's two (from the sums over the point's z).
-struct DzConst {
-    float ka, kb;
-};
-
-// Ackley's gradient factors from its sums s1 = sum z_j^2, s2 = sum sin^2(pi z_j).
-__device__ __forceinline__ DzConst ackley_const(float s1, float s2, int D) {
-    DzConst k;
-    const float Df = (float)D;
-    const float r = sqrtf(s1 / Df);
-    const float e1 = expm1_f(-0.2f * r) + 1.0f;
-    const float e2 = expm1_f(-2.0f * (s2 / Df)) + 1.0f;
-    k.ka = (r > 0.0f) ? (4.0f * e1) / (Df * r) : 0.0f;
-    k.kb = (6.28318548f * 2.71828175f / Df) * e2;
-    return k;
-}
-
-template <int FUNC>
-__device__ __forceinline__ DzConst dz_const(const float* z, int D) {
-    DzConst k{0.0f, 0.0f};
-    if constexpr (FUNC == F_ACKLEY) {
-        float s1 = 0.0f, s2 = 0.0f;
-        for (int j = 0; j < D; ++j) { s1 = s1 + z[j] * z[j]; s2 = s2 + sinpi_sq(z[j]); }
-        k = ackley_const(s1, s2, D);
-    }
-    return k;
-}
-
-// Griewank's factor cos(theta_j) = 1 - 2 sin^2(theta_j / 2), theta_j / (2 pi) = z_j tab[j]
-__device__ __forceinline__ float griewank_cos(float zj, float tj) { return 1.0f - 2.0f * sinpi_sq(zj * tj); }
-
-// d f / d z_j (0 for j >= D) of the point z; Griewank takes pre = prod_{k<j} cos(theta_k)
-// and suf = prod_{k>j} cos(theta_k), accumulated from the top.
+// d f / d z_j (0 for j >= D) of the point z in memory.
 template <int FUNC>
 __device__ __forceinline__ float dz_term(int j, const float* z, int D, const float* tab, const DzConst& kc, float pre,
                                          float suf) {
-    float v = 0.0f;
-    if (j < D) {
-        const float zj = z[j];
-        if constexpr (FUNC == F_SPHERE) v = 2.0f * zj;
-        else if constexpr (FUNC == F_ELLIPTIC) v = 2.0f * tab[j] * zj;
-        else if constexpr (FUNC == F_RASTRIGIN) v = 2.0f * zj + 62.8318531f * sin2pi(zj);
-        else if constexpr (FUNC == F_ACKLEY) v = kc.ka * zj + kc.kb * sin2pi(zj);
-        else if constexpr (FUNC == F_ROSENBROCK) {
-            if (j + 1 < D) v = 400.0f * zj * (zj * zj - z[j + 1]) + 2.0f * (zj - 1.0f);
-            if (j > 0) v = v - 200.0f * (z[j - 1] * z[j - 1] - zj);
-        } else if constexpr (FUNC == F_GRIEWANK) {
-            const float sn = sin2pi(zj * tab[j]);  // sin(theta_j)
-            v = zj / 2000.0f + pre * suf * sn * (6.28318548f * tab[j]);
-        } else if constexpr (FUNC == F_WEIERSTRASS) {
-            // sum_k 2^(1-k) pi 3^k sin(2 pi 3^k z), fractions of 3^k |z| as in the forward pass
-            const float a = __builtin_fabsf(zj);
-            float acc = 0.0f;
-            if (a < 8388608.0f) {
-                float c = 6.28318548f;  // 2 pi (1.5)^k
-                if (a < 2.32830644e-10f) {
-                    float p3 = 1.0f;
-                    for (int k = 0; k <= 20; ++k) {
-                        acc = fmaf(c, sin2pi(a * p3), acc);
-                        c = c * 1.5f;
-                        p3 = p3 * 3.0f;
-                    }
-                } else {
-                    const uint32_t u = __float_as_uint(a);
-                    const int ex = (int)((u >> 23) & 0xFFu) - 127;
-                    const uint64_t m = (uint64_t)((u & 0x007FFFFFu) | 0x00800000u);
-                    uint64_t y = m << (64 - (23 - ex));
-                    for (int k = 0; k <= 20; ++k) {
-                        const float r = (float)(uint32_t)(y >> 32) * 2.3283064365386963e-10f;
-                        acc = fmaf(c, sin2pi(r), acc);
-                        c = c * 1.5f;
-                        y = y + (y << 1);
-                    }
-                }
-            }
-            v = __builtin_copysignf(1.0f, zj) * acc;
-        } else if constexpr (FUNC == F_SCHWEFEL) {
-            const float sq = sqrtf(__builtin_fabsf(zj));
-            const float t = sq * 0.159154937f;
-            v = -(sin2pi(t) + 0.5f * sq * sin2pi(t + 0.25f));
-        }
-    }
-    return v;
-}
-
-// d f / d z_j of the lane's point for j = 2 s + h (the B-operand layout of the
-// second contraction), from the full z row in LDS.
-template <int KB, int FUNC>
-__device__ __forceinline__ void dfdz(float (&g)[4 * KB], const float* z, float* pre, int D, const float* tab, int h) {
-    constexpr int HS = 4 * KB;
-    if constexpr (FUNC == F_GRIEWANK) {
-        float p = 1.0f;  // prefix products
-        for (int j = 0; j < D; ++j) {
-            pre[j] = p;
-            p = p * griewank_cos(z[j], tab[j]);
-        }
-    }
-    const DzConst kc = dz_const<FUNC>(z, D);
-    float suf = 1.0f;  // Griewank suffix product, walked downwards
-    int jn = D - 1;
-#pragma unroll
-    for (int s = HS - 1; s >= 0; --s) {
-        const int j = 2 * s + h;
-        if constexpr (FUNC == F_GRIEWANK) {
-            while (jn > j) {
-                suf = suf * griewank_cos(z[jn], tab[jn]);
-                --jn;
-            }
-        }
-        g[s] = dz_term<FUNC>(j, z, D, tab, kc, (FUNC == F_GRIEWANK && j < D) ? pre[j] : 0.0f, suf);
-    }
+    if (j >= D) return 0.0f;
+    const bool ros = FUNC == F_ROSENBROCK;
+    return dz_elem<FUNC>(j, z[j], ros && j > 0 ? z[j - 1] : 0.0f, ros && j + 1 < D ? z[j + 1] : 0.0f, D, tab[j], kc, pre,
+                         suf);
 }
 
 // z rows of tile jt for the lane's column from w = x - o (the lane's parity half, in
@@ -1828,108 +1294,6 @@ __global__ __launch_bounds__(kThreads) EMTF_OCCUPANCY void island_persistent_ker
     }
 }
 
-template <int KB, int FUNC, bool ADJ>
-__global__ __launch_bounds__(2 * ObjShape<KB>::PB) void objective_kernel(ObjArgs a) {
-    using S = Shape<KB>;
-    constexpr int RS = S::RS, HS = S::HS, NT = S::NT, PB = ObjShape<KB>::PB, ZS = ObjShape<KB>::ZS;
-    extern __shared__ float smem[];
-    float* Q = smem;
-    float* o = Q + 32 * NT * RS;
-    float* tab = o + RS;
-    float* Zs = tab + 32 * NT;
-    float* Pre = Zs + PB * ZS;
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    const int D = a.dim;
-    for (int e = tid; e < 32 * NT * RS + RS + 32 * NT; e += nthr) smem[e] = 0.0f;
-    __syncthreads();
-    for (int e = tid; e < D * D; e += nthr) {
-        const int j = e / D, d = e - j * D;
-        Q[j * RS + (d & 1) * HS + (d >> 1)] = a.has_rot ? a.rot[e] : (j == d ? 1.0f : 0.0f);
-    }
-    for (int d = tid; d < D; d += nthr) {
-        o[(d & 1) * HS + (d >> 1)] = a.shift ? a.shift[d] : 0.0f;
-        tab[d] = a.tab[d];
-    }
-    __syncthreads();
-    const int wave = tid >> 6, lane = tid & 63, col = lane & 31, h = lane >> 5;
-    const int pt = blockIdx.x * PB + wave * 32 + col;
-    const bool valid = pt < a.n;
-    const float* xr = a.x + (int64_t)(valid ? pt : 0) * D;
-    float x[HS];
-#pragma unroll
-    for (int s = 0; s < HS; ++s) {
-        const int d = 2 * s + h;
-        x[s] = (d < D) ? xr[d] : 0.0f;
-    }
-    Geo g{};
-    g.D = D;
-    g.Dh = (D + 1) >> 1;
-    Lds L;
-    L.Q = Q;
-    L.o = o;
-    L.tab = tab;
-    if constexpr (!ADJ) {
-        const float f = evaluate_tile<KB, FUNC>(x, g, L, col, h);
-        if (valid && h == 0) a.f[pt] = f;
-    } else {
-        // z = Q (x - o) as in the forward pass, staged row-wise in LDS
-        f16v acc[NT];
-#pragma unroll
-        for (int jt = 0; jt < NT; ++jt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[jt][r] = 0.0f;
-#pragma unroll
-        for (int sb = 0; sb < KB; ++sb) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int s = 4 * sb + e;
-                const float w = x[s] - o[h * HS + s];
-#pragma unroll
-                for (int jt = 0; jt < NT; ++jt)
-                    acc[jt] = __builtin_amdgcn_mfma_f32_32x32x2f32(Q[(32 * jt + col) * RS + h * HS + s], w, acc[jt], 0, 0, 0);
-            }
-        }
-        float* zrow = Zs + (wave * 32 + col) * ZS;
-#pragma unroll
-        for (int jt = 0; jt < NT; ++jt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) zrow[32 * jt + 8 * (r >> 2) + 4 * h + (r & 3)] = acc[jt][r];
-        __syncthreads();
-        float dz[HS];
-        dfdz<KB, FUNC>(dz, zrow, Pre + (wave * 32 + col) * ZS, D, tab, h);
-        const float up = valid ? a.gf[pt] : 0.0f;
-#pragma unroll
-        for (int s = 0; s < HS; ++s) dz[s] = dz[s] * up;
-        // gx = Q^T dz: A[row d][k j] = Q[j][d]
-        f16v gacc[NT];
-#pragma unroll
-        for (int dt = 0; dt < NT; ++dt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) gacc[dt][r] = 0.0f;
-        const int dcol = col;  // lane's A row within the tile
-#pragma unroll
-        for (int s = 0; s < HS; ++s) {
-            const int j = 2 * s + h;
-#pragma unroll
-            for (int dt = 0; dt < NT; ++dt) {
-                const int d = 32 * dt + dcol;
-                const float qa = (j < 32 * NT) ? Q[j * RS + (d & 1) * HS + (d >> 1)] : 0.0f;
-                gacc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(qa, dz[s], gacc[dt], 0, 0, 0);
-            }
-        }
-        if (valid) {
-            float* gr = a.gx + (int64_t)pt * D;
-#pragma unroll
-            for (int dt = 0; dt < NT; ++dt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int d = 32 * dt + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (d < D) gr[d] = gacc[dt][r];
-                }
-        }
-    }
-}
-
 #if defined(EMTF_WIDE_NT)
 // ---------------------------------------------------------------------------
 // Wide tasks: dimensions up to 32 NT whose rows (or whose population) do not fit
@@ -2340,40 +1704,6 @@ __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     }
 }
 
-// emtf_objective_fwd for dimensions past the LDS evaluator's (D <= 32 NT): Q and the
-// points are read row-major from global memory, one gene pair per MFMA k-step in
-// increasing order with zero padding past D -- the engine evaluator's fma chains and
-// reductions, so the same bits.  128 points per workgroup, 32 per wave.
-template <int NT, int FUNC>
-__global__ __launch_bounds__(256) void objective_wide_kernel(ObjArgs a) {
-    __shared__ float o_s[32 * NT], tab_s[32 * NT];
-    const int tid = threadIdx.x, D = a.dim;
-    for (int d = tid; d < 32 * NT; d += 256) {
-        o_s[d] = (d < D && a.shift) ? a.shift[d] : 0.0f;
-        tab_s[d] = d < D ? a.tab[d] : 0.0f;
-    }
-    __syncthreads();
-    const int wave = tid >> 6, lane = tid & 63, col = lane & 31, h = lane >> 5;
-    const int pt = blockIdx.x * 128 + wave * 32 + col;
-    const bool valid = pt < a.n;
-    const float* xr = a.x + (int64_t)(valid ? pt : 0) * D;
-    f16v acc[NT];
-    zero_acc<NT>(acc);
-    const int Dh = (D + 1) >> 1;
-    for (int p = 0; p < Dh; ++p) {
-        const int d = 2 * p + h;
-        const float w = d < D ? xr[d] - o_s[d] : 0.0f;
-#pragma unroll
-        for (int jt = 0; jt < NT; ++jt) {
-            const int row = 32 * jt + col;
-            float q = 0.0f;
-            if (row < D && d < D) q = a.has_rot ? a.rot[(int64_t)row * D + d] : (row == d ? 1.0f : 0.0f);
-            acc[jt] = __builtin_amdgcn_mfma_f32_32x32x2f32(q, w, acc[jt], 0, 0, 0);
-        }
-    }
-    const float f = objective<NT, FUNC, true>(acc, D, tab_s, h);
-    if (valid && h == 0) a.f[pt] = f;
-}
 #endif  // EMTF_WIDE_NT
 
 }  // namespace emtf
@@ -2428,28 +1758,6 @@ extern "C" int EMTF_WNAME(emtf_wideq_lds_floats_nt, EMTF_WIDE_NT, a, EMTF_ALGO)(
 }
 #endif
 
-#if EMTF_ALGO == 0 && EMTF_WIDE_NT >= 5
-// emtf_objective_fwd for 128 < dim <= 32 NT (forward only)
-template <int FUNC>
-static hipError_t launch_obj_wide(const emtf::ObjArgs& a, hipStream_t stream) {
-    hipLaunchKernelGGL((emtf::objective_wide_kernel<EMTF_WIDE_NT, FUNC>), dim3((a.n + 127) / 128), dim3(256), 0, stream, a);
-    return hipGetLastError();
-}
-
-extern "C" int EMTF_WNAME(emtf_launch_objective_nt, EMTF_WIDE_NT, fw, d)(const emtf::ObjArgs* a, hipStream_t s) {
-    switch (a->func) {
-    case 0: return (int)launch_obj_wide<0>(*a, s);
-    case 1: return (int)launch_obj_wide<1>(*a, s);
-    case 2: return (int)launch_obj_wide<2>(*a, s);
-    case 3: return (int)launch_obj_wide<3>(*a, s);
-    case 4: return (int)launch_obj_wide<4>(*a, s);
-    case 5: return (int)launch_obj_wide<5>(*a, s);
-    case 6: return (int)launch_obj_wide<6>(*a, s);
-    case 7: return (int)launch_obj_wide<7>(*a, s);
-    }
-    return (int)hipErrorInvalidValue;
-}
-#endif
 #else
 #if !defined(EMTF_KB) || !defined(EMTF_ALGO)
 #error "compile island.hip with -DEMTF_KB=<gene blocks per half> -DEMTF_ALGO=<0|2>"
@@ -2504,35 +1812,6 @@ extern "C" int emtf_lds_floats_kb(int pop, int kb) { return emtf::lds_floats_kb(
 #endif
 
 #if EMTF_ALGO == 0
-// Objective kernels live in the DE translation unit of each KB.
-template <int FUNC, bool ADJ>
-static hipError_t launch_obj(const emtf::ObjArgs& a, hipStream_t stream) {
-    constexpr int KB = EMTF_KB;
-    auto k = &emtf::objective_kernel<KB, FUNC, ADJ>;
-    const int bytes = 4 * emtf::obj_lds_floats<KB>();
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (e != hipSuccess) return e;
-    constexpr int PB = emtf::ObjShape<KB>::PB;
-    hipLaunchKernelGGL(k, dim3((a.n + PB - 1) / PB), dim3(2 * PB), bytes, stream, a);
-    return hipGetLastError();
-}
-
-template <bool ADJ>
-static hipError_t launch_obj_any(const emtf::ObjArgs& a, hipStream_t s) {
-    switch (a.func) {
-    case 0: return launch_obj<0, ADJ>(a, s);
-    case 1: return launch_obj<1, ADJ>(a, s);
-    case 2: return launch_obj<2, ADJ>(a, s);
-    case 3: return launch_obj<3, ADJ>(a, s);
-    case 4: return launch_obj<4, ADJ>(a, s);
-    case 5: return launch_obj<5, ADJ>(a, s);
-    case 6: return launch_obj<6, ADJ>(a, s);
-    case 7: return launch_obj<7, ADJ>(a, s);
-    }
-    return hipErrorInvalidValue;
-}
-
 #define EMTF_OBJ_NAME2(a, b) a##b
 #define EMTF_OBJ_NAME(a, b) EMTF_OBJ_NAME2(a, b)
 
@@ -2557,9 +1836,6 @@ extern "C" int EMTF_OBJ_NAME(emtf_launch_polish_kb, EMTF_KB)(const emtf::EpochAr
     }
     hipLaunchKernelGGL(k, dim3(n), dim3(emtf::kThreads), lds_bytes, stream, *args, order);
     return (int)hipGetLastError();
-}
-extern "C" int EMTF_OBJ_NAME(emtf_launch_objective_kb, EMTF_KB)(const emtf::ObjArgs* a, int adjoint, hipStream_t s) {
-    return (int)(adjoint ? launch_obj_any<true>(*a, s) : launch_obj_any<false>(*a, s));
 }
 #endif
 #endif  // EMTF_WIDE_NT

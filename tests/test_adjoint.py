@@ -254,3 +254,46 @@ def test_gpu_transposed_rotation_view():
     a = forward_raw(3, x, q.t())
     b = forward_raw(3, x, q.t().contiguous())
     assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [1, 2, 8, 9, 16, 17, 32, 33, 64, 65, 96, 97, 127, 128, 129, 161, 224, 225, 256])
+def test_gpu_operator_tile_edges_bit_exact(oracle_mod, D):
+    """Forward and adjoint at the edges of the row tiles, gene strips and point tiles, on a
+    buffer that is only 4-byte aligned: the oracle's bits.  The upstream gradients are
+    powers of two, which scale the oracle's gradient exactly."""
+    from emtf.objective import adjoint_raw, forward_raw
+    for func, n in zip((0, 1, 2, 3, 4, 5, 6, 7, 1, 2, 4), (1, 31, 33, 65, 300, 40, 128, 7, 257, 129, 64)):
+        t = _task(func, D, n != 7, 700 + func)
+        x = _points(t, n, func + n, 1e-3 if func == 5 else 3.0)
+        print("case: tile edges D", D, "func", func, "n", n, flush=True)
+        flat = torch.empty(n * D + 1, dtype=torch.float32, device="cuda:0")
+        X = flat[1:].view(n, D)
+        X.copy_(torch.from_numpy(x))
+        rot, shift = _cuda(t.get("rot")), _cuda(t["shift"])
+        f = forward_raw(func, X, rot, shift).cpu().numpy()
+        assert np.array_equal(f.view(np.uint32), oracle_mod.eval32(t, x).view(np.uint32)), (func, n)
+        if D > 128:
+            continue
+        up = (2.0 ** (np.arange(n) % 5 - 2)).astype(np.float32)
+        g = adjoint_raw(func, X, _cuda(up), rot, shift).cpu().numpy()
+        ref = oracle_mod.grad32(t, x) * up[:, None]
+        assert np.array_equal(g.view(np.uint32), ref.view(np.uint32)), (func, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,n", [(2, 200001), (50, 140003), (100, 70001), (200, 66001)])
+def test_gpu_operator_many_tiles(oracle_mod, D, n):
+    """More point tiles than the grid holds at once, and a point with a NaN and one with an
+    infinity among them: every point equals the oracle's, the other points untouched."""
+    from emtf.objective import forward_raw
+    t = _task(3, D, True, 800)
+    x = _points(t, n, 1, 3.0)
+    x[n // 2, 0] = np.nan
+    x[n // 3, D - 1] = np.inf
+    print("case: many tiles D", D, "n", n, flush=True)
+    f = forward_raw(3, _cuda(x), _cuda(t["rot"]), _cuda(t["shift"])).cpu().numpy()
+    ref = oracle_mod.eval32(t, x)
+    assert np.array_equal(np.isnan(f), np.isnan(ref)) and np.isnan(ref).sum() <= 2
+    ok = ~np.isnan(ref)
+    assert np.array_equal(f[ok].view(np.uint32), ref[ok].view(np.uint32))
