@@ -11,9 +11,9 @@
 #include "../../include/emtf.h"
 #include "cvrp_types.h"
 
-extern "C" int emtf_cvrp_launch(const emtf::CvrpArgs* args, const int* order, int n_inst, int threads, int lds_bytes,
-                                int ring_bytes, hipStream_t stream);
-extern "C" int emtf_cvrp_lds_bytes(int n, int popP, int ring_bytes);
+extern "C" int emtf_cvrp_launch(const emtf::CvrpArgs* args, const int* order, int n_inst, int lds_bytes, int entry_bytes,
+                                hipStream_t stream);
+extern "C" int emtf_cvrp_lds_bytes(int n, int popP, int entry_bytes);
 extern "C" void emtf_set_error(const char* msg);
 
 namespace {
@@ -32,7 +32,7 @@ struct CvGroup {
 };
 
 struct emtf_cvrp_handle {
-    int T = 0, gen = 0, threads = 64, ring_bytes = 2;  // split ring entry size (2 or 4)
+    int T = 0, gen = 0, entry_bytes = 2;  // size of a split row entry (2 or 4)
     std::vector<CvGroup> groups;
     std::vector<hipStream_t> side;
     std::vector<hipEvent_t> ev_join;
@@ -82,7 +82,7 @@ static int cv_launch(emtf_cvrp_handle* h, int g0, int g1, int init, hipStream_t 
     }
     for (const CvGroup& g : h->groups) {
         hipStream_t q = g.stream == 0 ? s : h->side[g.stream - 1];
-        const int rc = emtf_cvrp_launch(&h->a, h->d_order + g.offset, g.count, h->threads, g.lds, h->ring_bytes, q);
+        const int rc = emtf_cvrp_launch(&h->a, h->d_order + g.offset, g.count, g.lds, h->entry_bytes, q);
         if (rc != 0) return cfail(EMTF_E_DEVICE, std::string("cvrp kernel launch: ") + hipGetErrorString((hipError_t)rc));
     }
     if (fork) {
@@ -120,7 +120,6 @@ int emtf_cvrp_create(const emtf_cvrp_instance* in, int32_t n_inst, const emtf_cv
     }
     emtf_cvrp_handle* h = new emtf_cvrp_handle();
     h->T = n_inst;
-    h->threads = (maxpop + 63) & ~63;
     h->inst.resize(n_inst);
     int64_t nt = 0, nc = 0, nd = 0, nx = 0, ne = 0;
     for (int t = 0; t < n_inst; ++t) {
@@ -158,12 +157,12 @@ int emtf_cvrp_create(const emtf_cvrp_instance* in, int32_t n_inst, const emtf_cv
         }
         off += (int64_t)S * S;
     }
-    // Split ring entries W_i + woff with W_i = V_i + d(0, t_i) - P_i: a label V_i never
+    // Split labels W_i + woff with W_i = V_i + d(0, t_i) - P_i: a label V_i never
     // exceeds the cost of serving each customer alone, sum_c 2 d(0, c), and a path prefix
     // P_i never exceeds (n - 1) dmax, so woff = (n - 1) dmax makes every entry non-negative
-    // and bounds it by woff + sum_c 2 d(0, c) + dmax.  The ring holds 16-bit entries when
-    // that bound fits for every instance, else W itself in 32 bits (woff = 0).
-    h->ring_bytes = 2;
+    // and bounds it by woff + sum_c 2 d(0, c) + dmax.  They are held in 16 bits when that
+    // bound fits for every instance, else in 32.
+    h->entry_bytes = 2;
     std::vector<int64_t> woffs(n_inst);
     for (int64_t t = 0, off = 0; t < n_inst; ++t) {
         const int S = in[t].n + 1;
@@ -171,17 +170,21 @@ int emtf_cvrp_create(const emtf_cvrp_instance* in, int32_t n_inst, const emtf_cv
         for (int c = 1; c < S; ++c) vbound += 2 * (int64_t)dist[off + c];
         for (int64_t e = 0; e < (int64_t)S * S; ++e) dmax = std::max<int64_t>(dmax, dist[off + e]);
         woffs[t] = (int64_t)(in[t].n - 1) * dmax;
-        if (woffs[t] + vbound + dmax >= 65536) h->ring_bytes = 4;
+        if (woffs[t] + vbound + dmax >= 65536) h->entry_bytes = 4;
         off += (int64_t)S * S;
     }
-    for (int t = 0; t < n_inst; ++t) h->inst[t].woff = h->ring_bytes == 2 ? (int32_t)woffs[t] : 0;
+    for (int t = 0; t < n_inst; ++t) h->inst[t].woff = (int32_t)woffs[t];
     // groups of equal occupancy (workgroups per CU from the LDS footprint), longest
     // instances first inside each group
     std::vector<int> occ(n_inst);
     for (int t = 0; t < n_inst; ++t) {
-        const int b = emtf_cvrp_lds_bytes(in[t].n, h->threads, h->ring_bytes);
-        if (b > kMaxLds) { cv_free(h); return cfail(EMTF_E_UNSUPPORTED, "instance exceeds LDS"); }
-        occ[t] = std::min(8, kMaxLds / b);
+        const int b = emtf_cvrp_lds_bytes(in[t].n, maxpop, h->entry_bytes);
+        // the engine's capacity: the population in whole waves, per individual two tours and
+        // 212 bytes (372 with 32-bit labels), and the nodes (the kernel itself needs less)
+        const int NP = (in[t].n + 3) & ~3, rows = (maxpop + 63) & ~63;
+        const int need = rows * (2 * NP + (h->entry_bytes == 2 ? 212 : 372)) + 6 * ((in[t].n + 4) & ~3);
+        if (b > kMaxLds || need > kMaxLds) { cv_free(h); return cfail(EMTF_E_UNSUPPORTED, "instance exceeds LDS"); }
+        occ[t] = std::min(4, kMaxLds / b);  // 512 threads: four workgroups fill a CU
     }
     std::vector<int> order(n_inst);
     for (int t = 0; t < n_inst; ++t) order[t] = t;
@@ -193,7 +196,7 @@ int emtf_cvrp_create(const emtf_cvrp_instance* in, int32_t n_inst, const emtf_cv
         CvGroup g;
         g.offset = r;
         while (r < n_inst && occ[order[r]] == occ[order[g.offset]]) {
-            g.lds = std::max(g.lds, emtf_cvrp_lds_bytes(in[order[r]].n, h->threads, h->ring_bytes));
+            g.lds = std::max(g.lds, emtf_cvrp_lds_bytes(in[order[r]].n, maxpop, h->entry_bytes));
             ++r;
         }
         g.count = r - g.offset;
@@ -242,6 +245,7 @@ int emtf_cvrp_create(const emtf_cvrp_instance* in, int32_t n_inst, const emtf_cv
     a.n_islands = nis;
     a.migrate_interval = prm->migrate_interval;
     a.migrate_count = prm->migrate_count;
+    a.popP = maxpop;
     a.seed_lo = (uint32_t)prm->seed;
     a.seed_hi = (uint32_t)(prm->seed >> 32);
     int rc = cv_launch(h, 0, 0, 1, nullptr);

@@ -22,6 +22,7 @@ struct CvrpArgs {
     const uint8_t* dem;
     float p_swap, p_2opt;
     int32_t n_islands, migrate_interval, migrate_count;
+    int32_t popP;  // rows of the per-individual arrays in LDS: the largest population
     uint32_t seed_lo, seed_hi;
 };
 

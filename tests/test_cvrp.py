@@ -200,3 +200,35 @@ def test_gpu_cvrp_full_size_properties(oracle_mod):
         for k in range(0, ins["pop"], 9):
             assert sorted(tours[k].tolist()) == list(range(1, ins["n"] + 1))
             assert costs[k] == oracle_mod.cvrp_split(tours[k], dist, dem, ins["capacity"]), (i, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pop,n_islands", [(2, 1), (66, 1), (130, 2), (200, 4)])
+def test_gpu_cvrp_chunk_edges(oracle_mod, pop, n_islands):
+    """Tours at the edges of the 64-position chunks, populations that do not fill the
+    64-individual passes, and capacities whose windows end around the 16 positions held in
+    registers, the 32 of the search's first round and the longest route (63): bit-exact
+    with the oracle; best() is the first of the smallest costs."""
+    from emtf.cvrp import CvrpEngine
+    rng = np.random.default_rng(pop)
+    ns = (2, 3, 63, 64, 65, 127, 128, 129, 160) if pop > 130 else (2, 4, 16, 17, 64, 65, 128, 129, 191, 192, 193)
+    inst = []
+    for n, cap in zip(ns, (15, 16, 17, 31, 32, 33, 63, 50, 12, 40, 62)):
+        xy = np.vstack([[50, 50], rng.integers(0, 101, (n, 2))]).astype(np.int32)
+        dem = np.concatenate([[0], np.ones(n) if cap != 50 else rng.integers(1, 11, n)]).astype(np.int32)
+        inst.append(dict(n=n, capacity=cap, pop=pop, xy=xy, demand=dem))
+    params = dict(p_swap=0.4, p_2opt=0.4, n_islands=n_islands, migrate_interval=2 if n_islands > 1 else 0,
+                  migrate_count=1 if n_islands > 1 else 0, seed=6)
+    print("case: cvrp edges pop", pop, flush=True)
+    gpu = CvrpEngine(inst, **params)
+    orc = oracle_mod.CvrpEngine(inst, **params)
+    gpu.run(9)
+    orc.run(9)
+    cost, tour = gpu.best()
+    for i in range(len(inst)):
+        tg, cg = gpu.population(i)
+        to, co = orc.population(i)
+        assert np.array_equal(cg, co), i
+        assert np.array_equal(tg, to), i
+        b = int(np.argmin(co))
+        assert cost[i] == co[b] and np.array_equal(tour[i, :inst[i]["n"]], to[b]) and not tour[i, inst[i]["n"]:].any()
