@@ -568,7 +568,49 @@ __global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4)))
     for (int i = tid; i < pop; i += kCvThreads) a.cost[cd.cost_off + i] = L.cost[i];
 }
 
+// Best individual of every instance (the first of the smallest cost), one wave each: its cost
+// and its tour (rows of `stride` bytes), written straight into pinned host memory.
+__global__ __launch_bounds__(64) void cvrp_best_kernel(const CvrpDev* __restrict__ inst, const int32_t* __restrict__ cost,
+                                                       const uint8_t* __restrict__ tours, int stride,
+                                                       int32_t* __restrict__ out_cost, uint8_t* __restrict__ out_tour) {
+    const int t = blockIdx.x, lane = threadIdx.x;
+    const CvrpDev cd = inst[t];
+    int32_t bc = 0x7FFFFFFF;
+    int bi = 0;
+    for (int i = lane; i < cd.pop; i += 64) {
+        const int32_t c = cost[cd.cost_off + i];
+        if (c < bc) {
+            bc = c;
+            bi = i;
+        }
+    }
+#pragma unroll
+    for (int w = 32; w >= 1; w >>= 1) {
+        const int32_t oc = __shfl_xor(bc, w);
+        const int oi = __shfl_xor(bi, w);
+        if (oc < bc || (oc == bc && oi < bi)) {
+            bc = oc;
+            bi = oi;
+        }
+    }
+    if (lane == 0) out_cost[t] = bc;
+    const uint8_t* src = tours + cd.tour_off + (int64_t)bi * cd.n;
+    uint8_t* dst = out_tour + (int64_t)t * stride;
+    for (int k = 4 * lane; k < cd.n; k += 256) {  // stride is a multiple of 4
+        uint32_t v = 0;
+        for (int b = 0; b < 4; ++b) v |= (uint32_t)(k + b < cd.n ? src[k + b] : 0) << (8 * b);
+        *reinterpret_cast<uint32_t*>(dst + k) = v;
+    }
+}
+
 }  // namespace emtf
+
+extern "C" int emtf_cvrp_launch_best(const emtf::CvrpDev* inst, int n_inst, const int32_t* cost, const uint8_t* tours,
+                                     int stride, int32_t* out_cost, uint8_t* out_tour, hipStream_t stream) {
+    hipLaunchKernelGGL(emtf::cvrp_best_kernel, dim3(n_inst), dim3(64), 0, stream, inst, cost, tours, stride, out_cost,
+                       out_tour);
+    return (int)hipGetLastError();
+}
 
 extern "C" int emtf_cvrp_lds_bytes(int n, int popP, int entry_bytes) {
     return emtf::cvrp_lds_bytes(n, popP, entry_bytes);

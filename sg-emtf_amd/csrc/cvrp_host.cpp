@@ -13,6 +13,8 @@
 
 extern "C" int emtf_cvrp_launch(const emtf::CvrpArgs* args, const int* order, int n_inst, int lds_bytes, int entry_bytes,
                                 hipStream_t stream);
+extern "C" int emtf_cvrp_launch_best(const emtf::CvrpDev* inst, int n_inst, const int32_t* cost, const uint8_t* tours,
+                                     int stride, int32_t* out_cost, uint8_t* out_tour, hipStream_t stream);
 extern "C" int emtf_cvrp_lds_bytes(int n, int popP, int entry_bytes);
 extern "C" void emtf_set_error(const char* msg);
 
@@ -46,6 +48,8 @@ struct emtf_cvrp_handle {
     int32_t* d_cost = nullptr;
     uint32_t* d_xy = nullptr;
     uint8_t* d_dem = nullptr;
+    int32_t* best = nullptr;  // pinned: every instance's best cost, then its tour (rows of best_stride)
+    int best_stride = 0;
     hipStream_t stream = nullptr;
 };
 
@@ -57,6 +61,7 @@ static void cv_free(emtf_cvrp_handle* h) {
     (void)hipFree(h->d_cost);
     (void)hipFree(h->d_xy);
     (void)hipFree(h->d_dem);
+    if (h->best) (void)hipHostFree(h->best);
     for (hipStream_t s : h->side) (void)hipStreamDestroy(s);
     for (hipEvent_t e : h->ev_join) (void)hipEventDestroy(e);
     if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
@@ -233,6 +238,11 @@ int emtf_cvrp_create(const emtf_cvrp_instance* in, int32_t n_inst, const emtf_cv
         cv_free(h);
         return cfail(EMTF_E_DEVICE, "hipMemcpy failed");
     }
+    for (int t = 0; t < n_inst; ++t) h->best_stride = std::max(h->best_stride, (in[t].n + 3) & ~3);
+    if (!ok(hipHostMalloc((void**)&h->best, (size_t)n_inst * (4 + h->best_stride), hipHostMallocDefault))) {
+        cv_free(h);
+        return cfail(EMTF_E_NOMEM, "hipHostMalloc failed");
+    }
     emtf::CvrpArgs& a = h->a;
     a.inst = h->d_inst;
     a.n_inst = n_inst;
@@ -296,20 +306,15 @@ int emtf_cvrp_get_population(emtf_cvrp_handle* h, int32_t i, uint8_t* tours, int
 
 int emtf_cvrp_get_best(emtf_cvrp_handle* h, int32_t* cost, uint8_t* tour, int32_t stride) {
     if (!h) return cfail(EMTF_E_INVALID, "handle is NULL");
-    std::vector<int32_t> c;
-    std::vector<uint8_t> t;
+    for (int i = 0; tour && i < h->T; ++i)
+        if (stride < h->inst[i].n) return cfail(EMTF_E_INVALID, "stride < n");
+    uint8_t* bt = reinterpret_cast<uint8_t*>(h->best + h->T);
+    const int rc = emtf_cvrp_launch_best(h->d_inst, h->T, h->d_cost, h->d_tours, h->best_stride, h->best, bt, h->stream);
+    if (rc != 0) return cfail(EMTF_E_DEVICE, std::string("best: ") + hipGetErrorString((hipError_t)rc));
+    if (hipStreamSynchronize(h->stream) != hipSuccess) return cfail(EMTF_E_DEVICE, "hipStreamSynchronize");
     for (int i = 0; i < h->T; ++i) {
-        const emtf::CvrpDev& d = h->inst[i];
-        if (tour && stride < d.n) return cfail(EMTF_E_INVALID, "stride < n");
-        c.resize(d.pop);
-        t.resize((size_t)d.pop * d.n);
-        const int rc = emtf_cvrp_get_population(h, i, tour ? t.data() : nullptr, c.data());
-        if (rc != EMTF_OK) return rc;
-        int best = 0;
-        for (int k = 1; k < d.pop; ++k)
-            if (c[k] < c[best]) best = k;
-        if (cost) cost[i] = c[best];
-        if (tour) std::memcpy(tour + (size_t)i * stride, t.data() + (size_t)best * d.n, d.n);
+        if (cost) cost[i] = h->best[i];
+        if (tour) std::memcpy(tour + (size_t)i * stride, bt + (size_t)i * h->best_stride, h->inst[i].n);
     }
     return EMTF_OK;
 }
