@@ -18,9 +18,12 @@ LIB = os.path.join(HERE, "libemtf.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -ffp-contract=off: the arithmetic contract forbids implicit fma contraction.
+# -pragma-unroll-threshold: the per-row epilogues of 5 to 8 row tiles are unrolled in full (a
+# loop left over indexes the accumulators, which puts them in scratch memory).
 # -packed-fp32-ops: keep the device compiler away from v_pk_{add,mul,fma}_f32.
 COMMON = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-ffp-contract=off", "-fPIC",
-          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function"]
+          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function",
+          "-mllvm", "-pragma-unroll-threshold=65536"]
 # (gene blocks per parity half KB: dims <= 8 KB; algorithm family: 0 = DE, 2 = GA)
 VARIANTS = [(kb, al) for kb in (2, 4, 7, 8, 12, 13, 16) for al in (0, 2)]
 # wide kernel: (32-row tiles NT: dims <= 32 NT, rows in global memory; algorithm family)

@@ -188,7 +188,7 @@ __device__ __forceinline__ float objective(const f16v (&acc)[NT], int D, const f
                         z = e == 3 ? acc[jt][4 * g + 3] : z;
                         const float a = __builtin_fabsf(z);
                         if (z != z || (a > 0.0f && a < 2.32830644e-10f)) {
-                            const float r = weier_term(z);
+                            const float r = weier_rare(z);
 #pragma unroll
                             for (int f = 0; f < 4; ++f) v[f] = e == f ? r : v[f];
                         }
@@ -382,7 +382,7 @@ __device__ __forceinline__ void tile_vals(const f16v& acc, int jt, int D, const 
                     z = e == 3 ? acc[4 * g + 3] : z;
                     const float a = __builtin_fabsf(z);
                     if (z != z || (a > 0.0f && a < 2.32830644e-10f)) {
-                        const float r = weier_term(z);
+                        const float r = weier_rare(z);
 #pragma unroll
                         for (int f = 0; f < 4; ++f) v[f] = e == f ? r : v[f];
                     }

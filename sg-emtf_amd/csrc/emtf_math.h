@@ -241,24 +241,29 @@ __device__ __forceinline__ float weier_core(float a, bool ok) {
     return ok ? acc : 0.0f;
 }
 
-__device__ __forceinline__ float weier_term(float z) {
+// The term for a NaN or 0 < |z| < 2^-32, which weier_core leaves out: there 3^k |z| < 1 needs
+// no reduction.  Rolled (p <- 3 p gives the correctly rounded powers of three), so that the
+// kernels that inline it per group of rows stay small: unrolled, 16 groups of it outgrew the
+// unrolling limit and the accumulators went to scratch memory.
+__device__ __forceinline__ float weier_rare(float z) {
     if (z != z) return z;
     const float a = __builtin_fabsf(z);
-    float acc = 0.0f;
-    if (a >= 8388608.0f) return 0.0f;
-    if (a < 2.32830644e-10f) {
-        // 3^k as binary32 (exact for k <= 15, correctly rounded above); 3^k a < 1
-        constexpr float P3F[21] = {1.f, 3.f, 9.f, 27.f, 81.f, 243.f, 729.f, 2187.f, 6561.f, 19683.f,
-                                   59049.f, 177147.f, 531441.f, 1594323.f, 4782969.f, 14348907.f,
-                                   43046721.f, 129140163.f, 387420489.f, 1162261467.f, 3486784401.f};
-#pragma unroll
-        for (int k = 0; k <= 20; ++k) {
-            const float r = a * P3F[k];
-            const float sp = sinpi_half(__builtin_fminf(r, 1.0f - r));
-            acc = fmaf(pow2i(1 - k), sp * sp, acc);
-        }
-        return acc;
+    float acc = 0.0f, p3 = 1.0f, w = 2.0f;
+#pragma unroll 1
+    for (int k = 0; k <= 20; ++k) {
+        const float r = a * p3;
+        const float sp = sinpi_half(__builtin_fminf(r, 1.0f - r));
+        acc = fmaf(w, sp * sp, acc);
+        p3 = p3 * 3.0f;
+        w = w * 0.5f;
     }
+    return acc;
+}
+
+__device__ __forceinline__ float weier_term(float z) {
+    const float a = __builtin_fabsf(z);
+    if (a >= 8388608.0f) return 0.0f;
+    if (z != z || a < 2.32830644e-10f) return weier_rare(z);
     return weier_core(a, true);
 }
 
