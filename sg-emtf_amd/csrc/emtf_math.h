@@ -26,26 +26,65 @@ enum Purpose : uint32_t {
 
 struct U4 { uint32_t x, y, z, w; };
 
-__device__ __forceinline__ U4 philox(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
-                                     uint32_t k0, uint32_t k1) {
-    // the key schedule is re-derived per block with two scalar adds a round; without
+// N blocks whose counters share their last two words, round by round together: one key
+// schedule serves them all and their chains overlap.
+template <int N>
+__device__ __forceinline__ void philox_blocks(U4 (&out)[N], const uint32_t (&c0_)[N], const uint32_t (&c1_)[N],
+                                              uint32_t c2_, uint32_t c3_, uint32_t k0, uint32_t k1) {
+    // the key schedule is re-derived per call with two scalar adds a round; without
     // this the compiler keeps all twenty round keys live across the generation loop,
     // where they spill and come back as VALU lane reads
     asm volatile("" : "+s"(k0), "+s"(k1));
+    uint32_t c0[N], c1[N], c2[N], c3[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        c0[i] = c0_[i];
+        c1[i] = c1_[i];
+        c2[i] = c2_;
+        c3[i] = c3_;
+    }
+    // The counter's lane-varying word (c1) reaches the other words in round 3: the first three
+    // rounds keep their uniform halves on the scalar unit (the key and a uniform word are
+    // joined first), from then on each new word is one three-input xor (v_bitop3_b32, 4
+    // cycles with its scalar key operand where two xors take 2 + 4).
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
-        const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
-        const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-        const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
-        const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
-        c1 = (uint32_t)p1;
-        c3 = (uint32_t)p0;
-        c0 = n0;
-        c2 = n2;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const uint64_t p0 = (uint64_t)0xD2511F53u * c0[i];
+            const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2[i];
+            const uint32_t h0 = (uint32_t)(p0 >> 32), h1 = (uint32_t)(p1 >> 32);
+            uint32_t n0, n2;
+            if (r == 0) {
+                n0 = (h1 ^ k0) ^ c1[i];
+                n2 = (h0 ^ k1) ^ c3[i];
+            } else if (r == 1) {
+                n0 = (h1 ^ k0) ^ c1[i];
+                n2 = (c3[i] ^ k1) ^ h0;
+            } else if (r == 2) {
+                n0 = (c1[i] ^ k0) ^ h1;
+                n2 = (h0 ^ k1) ^ c3[i];
+            } else {
+                n0 = __builtin_amdgcn_bitop3_b32(h1, c1[i], k0, 0x96);
+                n2 = r == 3 ? (c3[i] ^ k1) ^ h0 : __builtin_amdgcn_bitop3_b32(h0, c3[i], k1, 0x96);
+            }
+            c1[i] = (uint32_t)p1;
+            c3[i] = (uint32_t)p0;
+            c0[i] = n0;
+            c2[i] = n2;
+        }
         k0 += 0x9E3779B9u;
         k1 += 0xBB67AE85u;
     }
-    return U4{c0, c1, c2, c3};
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = U4{c0[i], c1[i], c2[i], c3[i]};
+}
+
+__device__ __forceinline__ U4 philox(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1) {
+    U4 out[1];
+    const uint32_t a0[1] = {c0}, a1[1] = {c1};
+    philox_blocks<1>(out, a0, a1, c2, c3, k0, k1);
+    return out[0];
 }
 
 struct Rng {
@@ -53,6 +92,18 @@ struct Rng {
     __device__ __forceinline__ U4 block(uint32_t gen, uint32_t purpose, uint32_t index, uint32_t sub,
                                         uint32_t blk) const {
         return philox(blk, (purpose << 24) | ((sub & 0xFFu) << 16) | (index & 0xFFFFu), gen, task, k0, k1);
+    }
+    // blocks blk .. blk + N - 1 of one address
+    template <int N>
+    __device__ __forceinline__ void blocks(U4 (&out)[N], uint32_t gen, uint32_t purpose, uint32_t index, uint32_t sub,
+                                           uint32_t blk) const {
+        uint32_t c0[N], c1[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            c0[i] = blk + (uint32_t)i;
+            c1[i] = (purpose << 24) | ((sub & 0xFFu) << 16) | (index & 0xFFFFu);
+        }
+        philox_blocks<N>(out, c0, c1, gen, task, k0, k1);
     }
     __device__ __forceinline__ uint32_t word(uint32_t gen, uint32_t purpose, uint32_t index, uint32_t sub,
                                              uint32_t w) const {

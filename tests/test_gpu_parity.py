@@ -431,3 +431,15 @@ def test_full_size_uneven_properties():
     assert sum(tasks[t]["dim"] > 128 for t in ids) > 30
     _fitness_matches_fresh_evaluation(gpu, tasks, ids)
     gpu.close()
+
+
+# ---- the kernels' dispatch edges
+@pytest.mark.parametrize("CR", [0.0, 1.0e-5, 0.5, 1.0])
+def test_crossover_thresholds(oracle_mod, CR):
+    """CR at the ends of its range: a threshold of zero (only jrand crosses) and one above
+    every 16-bit draw, in the LDS and the wide kernel."""
+    tasks = tg.benchmark_tasks(4, 50, 64, rotate=True, seed=51) + tg.benchmark_tasks(2, 131, 40, rotate=True, seed=52)
+    gpu, orc = _pair(tasks, oracle_mod, seed=3, CR=CR)
+    gpu.run(6)
+    orc.run(6)
+    _compare(gpu, orc, f"CR {CR}")
