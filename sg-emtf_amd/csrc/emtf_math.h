@@ -239,6 +239,74 @@ __device__ __forceinline__ float pow_f(float x, float y) {
     return exp2_f(ly);
 }
 
+// ---- the same functions on the arguments the GA's operators nearly always have ------------
+// Quotients below: a reciprocal estimate, one Newton step, then Markstein's correction of
+// the quotient by its exact remainder (P. Markstein, "Computation of elementary functions on the
+// IBM RISC System/6000 processor", 1990): correctly rounded on the stated ranges, in 18 cycles
+// where the general sequence (scaling, fix-up) takes over 40.
+
+// (m - 1) / (m + 1) for m in (0.7071, 1.4143): equal to the division for every such m
+// (all 8.4 million binary32 values compared).
+__device__ __forceinline__ float ratio_near1(float m) {
+    const float a = m - 1.0f, b = m + 1.0f;
+    float r = __builtin_amdgcn_rcpf(b);
+    r = fmaf(fmaf(-b, r, 1.0f), r, r);
+    const float q = a * r;
+    return fmaf(fmaf(-b, q, a), r, q);
+}
+
+// 1 / b for b = k 2^-24, 1 <= k <= 2^23: equal to the division for every such b (all compared).
+__device__ __forceinline__ float recip24(float b) {
+    float r = __builtin_amdgcn_rcpf(b);
+    r = fmaf(fmaf(-b, r, 1.0f), r, r);
+    return fmaf(fmaf(-b, r, 1.0f), r, r);
+}
+
+// a / b with y = 1 / b correctly rounded, b and a / b far from the ends of the exponent range
+// (or a = 0): the first correction leaves at most one unit of error, the second is Markstein's.
+__device__ __forceinline__ float quot_by(float a, float b, float y) {
+    float q = a * y;
+    q = fmaf(fmaf(-b, q, a), y, q);
+    return fmaf(fmaf(-b, q, a), y, q);
+}
+
+// log2_f for a positive normal x (a finite value for any other): the exponent and the
+// mantissa in [0.7071, 1.4142] by one addition, the polynomial as there.
+__device__ __forceinline__ float log2_normal(float x) {
+    const uint32_t u = __float_as_uint(x);
+    const uint32_t t = u + 0x004AFB0Cu;  // carries into the exponent where the mantissa exceeds 1.41421354
+    const float e = (float)((int32_t)t >> 23) - 127.0f;
+    const float m = __uint_as_float(u - (t & 0xFF800000u) + 0x3F800000u);
+    const float s = ratio_near1(m);
+    const float x2 = s * s;
+    float p = 2.828850150e-01f;
+    p = fmaf(p, x2, 3.199068010e-01f);
+    p = fmaf(p, x2, 4.122092128e-01f);
+    p = fmaf(p, x2, 5.770779252e-01f);
+    p = fmaf(p, x2, 9.617967010e-01f);
+    p = fmaf(p, x2, 2.885390043e+00f);
+    const float tt = s * p;
+    return e + tt;
+}
+
+// exp2_f for |y| <= 10^6: one scaling by 2^n, rounded (to a subnormal, zero or infinity) once.
+__device__ __forceinline__ float exp2_mid(float y) {
+    const float n = __builtin_rintf(y);
+    const float f = y - n;
+    float p = 1.530369991e-05f;
+    p = fmaf(p, f, 1.546972926e-04f);
+    p = fmaf(p, f, 1.333347871e-03f);
+    p = fmaf(p, f, 9.618025273e-03f);
+    p = fmaf(p, f, 5.550410971e-02f);
+    p = fmaf(p, f, 2.402265072e-01f);
+    p = fmaf(p, f, 6.931471825e-01f);
+    p = fmaf(p, f, 1.000000000e+00f);
+    return __builtin_amdgcn_ldexpf(p, (int)n);
+}
+
+// pow_f for a positive normal x and |y| <= 1000.
+__device__ __forceinline__ float pow_mid(float x, float y) { return exp2_mid(y * log2_normal(x)); }
+
 // sin^2(pi t) = x Q_d(x), x = t^2, t in [-1/2, 1/2]: Q_d of degree d fitted to
 // sin^2(pi sqrt(x)) / x on [0, 1/4] by least squares reweighted toward the minimax of the
 // relative error (Lawson's iteration; oracle/fit_coeffs.py); largest relative error of the

@@ -443,3 +443,18 @@ def test_crossover_thresholds(oracle_mod, CR):
     gpu.run(6)
     orc.run(6)
     _compare(gpu, orc, f"CR {CR}")
+
+
+@pytest.mark.parametrize("box", [(-100.0, 100.0), (0.0, 1.0), (-1.0, 0.0), (1.0, 1.0000001), (1e-20, 1e-18),
+                                 (-1e12, 3e15), (-3e-10, 5e-10)])
+@pytest.mark.parametrize("eta_c, eta_m, pm", [(2.0, 5.0, 1.0), (0.0, 0.0, 0.5), (20.0, 2000.0, 1.0)])
+def test_ga_boxes_and_exponents(oracle_mod, box, eta_c, eta_m, pm):
+    """The GA's operators inside and outside the range of their quick forms: boxes that touch
+    zero, one unit wide, far from one in magnitude; large and zero distribution indices."""
+    tasks = tg.benchmark_tasks(3, 21, 64, rotate=True, seed=53) + tg.benchmark_tasks(1, 140, 32, rotate=True, seed=54)
+    for t in tasks:
+        t["lo"], t["hi"] = box
+    gpu, orc = _pair(tasks, oracle_mod, seed=4, algo=emtf.GA_SBX_PM, eta_c=eta_c, eta_m=eta_m, pm=pm)
+    gpu.run(6)
+    orc.run(6)
+    _compare(gpu, orc, f"GA box {box} eta {eta_c}, {eta_m}")
