@@ -434,6 +434,21 @@ def test_full_size_uneven_properties():
 
 
 # ---- the kernels' dispatch edges
+@pytest.mark.parametrize("algo", [emtf.DE_RAND_1_BIN, emtf.GA_SBX_PM])
+@pytest.mark.parametrize("pop", [128, 160])
+def test_gene_block_edges(oracle_mod, algo, pop):
+    """Dimensions on both sides of every gene block that a kernel build skips, of its row
+    tiles and of the builds themselves (the last two read Q from global memory), at four
+    tiles (mates drawn for two generations at once) and five."""
+    dims = [8, 9, 16, 17, 24, 25, 32, 33, 37, 40, 41, 56, 57, 64, 65, 72, 73, 96, 97, 100, 104, 105, 112, 113, 127, 128]
+    tasks = tg.benchmark_tasks(len(dims), 0, pop, rotate=True, seed=50, dims=dims)
+    gpu, orc = _pair(tasks, oracle_mod, seed=2, tune=1, algo=algo, transfer_interval=3, transfer_count=2)
+    for step in (3, 4):
+        gpu.run(step)
+        orc.run(step)
+        _compare(gpu, orc, f"gene blocks algo {algo} gen {orc.generation}")
+
+
 @pytest.mark.parametrize("CR", [0.0, 1.0e-5, 0.5, 1.0])
 def test_crossover_thresholds(oracle_mod, CR):
     """CR at the ends of its range: a threshold of zero (only jrand crosses) and one above
