@@ -73,9 +73,8 @@ typedef struct emtf_params {
                                    decisions are kept for later creates of a batch with the same
                                    launch units: in memory for the process, and in the file the
                                    environment variable EMTF_TUNE_CACHE names, if set); 1: off;
-                                   2: the first alternative variant where one exists (the wide
-                                   kernel, or its 512-thread build); 3: the wide kernel with Q in
-                                   LDS where it fits (2 and 3 for testing) */
+                                   2 and 3: the alternative variant where one exists (the wide
+                                   kernel, for tasks that the LDS kernel holds; for testing) */
     int32_t formulas;           /* EMTF_FORMULAS_*: which formulas evaluate the objectives */
     int32_t admission;          /* EMTF_ADMIT_*: when tasks start */
 } emtf_params;

@@ -30,8 +30,9 @@ constexpr bool zero_term_at_zero() {
 }
 
 // The objective's terms and final combination in split form, for the polish's line search
-// (terms of a row tile computed apart from the running sums): the same operations, in the
-// same order, as objective() below, which keeps them inline for the epoch kernels' code.
+// and the wide kernel's row tiles on several waves (terms of a row tile computed apart from
+// the running sums): the same operations, in the same order, as objective() below, which
+// keeps them inline for the epoch kernels' code.
 //
 // Rosenbrock's term of row j (z = z_j, zn = z_{j+1}); it counts when row j + 1 exists.
 __device__ __forceinline__ float rosen_val(float z, float zn) {
@@ -44,11 +45,11 @@ __device__ __forceinline__ float rosen_val(float z, float zn) {
     return t1 + b2;
 }
 
-// The term values of row j of every textbook objective but Rosenbrock (v2: Ackley's
-// cosine term, Griewank's 2 sin^2); the Weierstrass term only for rows j < Dm (0 otherwise).
+// The term values of row j of every objective but Rosenbrock and (textbook) Weierstrass (v2:
+// Ackley's cosine term, Griewank's 2 sin^2 or the reference's factor); the Weierstrass terms
+// only for rows j < Dm (0 otherwise).
 template <int FUNC>
 __device__ __forceinline__ void row_vals(float z, int j, int Dm, const float* tab, float& v1, float& v2) {
-    static_assert(FUNC <= F_ELLIPTIC, "textbook objectives only");
     if constexpr (FUNC == F_SPHERE) {
         v1 = z * z;
     } else if constexpr (FUNC == F_ELLIPTIC) {
@@ -71,7 +72,34 @@ __device__ __forceinline__ void row_vals(float z, int j, int Dm, const float* ta
         const float sq = sqrtf(__builtin_fabsf(z));
         const float tv = sq * 0.159154937f;
         v1 = z * sin2pi(tv);
+    } else if constexpr (FUNC == F_REF_ACKLEY) {
+        v1 = z * z;
+        const float tz = 2.0f * z;
+        v2 = cospi_f(tz);
+    } else if constexpr (FUNC == F_REF_RASTRIGIN) {
+        const float zz = z * z;
+        const float tz = 2.0f * z;
+        const float c = cospi_f(tz);
+        const float t = 10.0f * c;
+        const float v = zz - t;
+        v1 = v + 10.0f;
+    } else if constexpr (FUNC == F_REF_GRIEWANK) {
+        v1 = z * z;
+        const float q = z / tab[j];
+        const float tq = q * 0.159154937f;
+        const float t = 2.0f * sinpi_sq(tq);
+        v2 = 1.0f - t;
+    } else if constexpr (FUNC == F_REF_WEIERSTRASS) {
+        v1 = 0.0f;
+        if (j < Dm) v1 = weier_ref_term(z);
     }
+}
+
+// The running sums' start (s2: the reference Griewank's product).
+template <int FUNC>
+__device__ __forceinline__ void sums_start(float& s1, float& s2) {
+    s1 = 0.0f;
+    s2 = (FUNC == F_REF_GRIEWANK) ? 1.0f : 0.0f;
 }
 
 // Adds one row's term values into the lane's sums (s2: Ackley's cosine sum, Griewank's
@@ -80,8 +108,10 @@ template <int FUNC>
 __device__ __forceinline__ void row_sum(float v1, float v2, bool in, float& s1, float& s2) {
     if (!in) return;
     s1 = s1 + v1;
-    if constexpr (FUNC == F_ACKLEY) {
+    if constexpr (FUNC == F_ACKLEY || FUNC == F_REF_ACKLEY) {
         s2 = s2 + v2;
+    } else if constexpr (FUNC == F_REF_GRIEWANK) {
+        s2 = s2 * v2;
     } else if constexpr (FUNC == F_GRIEWANK) {
         const float om = 1.0f - s2;
         const float aq = v2 * om;
@@ -90,10 +120,9 @@ __device__ __forceinline__ void row_sum(float v1, float v2, bool in, float& s1, 
 }
 
 // The fitness from the two halves' sums (lane h holds its half's s1, s2; the other
-// half's come over the cross-half shuffle), textbook objectives.
+// half's come over the cross-half shuffle).
 template <int FUNC>
 __device__ __forceinline__ float objective_tail(float s1, float s2, int D, const float* tab, int h) {
-    static_assert(FUNC <= F_ELLIPTIC, "textbook objectives only");
     const float o1 = __shfl_xor(s1, 32);
     const float S = s1 + o1;  // A + B (commutative)
     const float Df = (float)D;
@@ -121,6 +150,31 @@ __device__ __forceinline__ float objective_tail(float s1, float s2, int D, const
         // the constant from the task table: 418.982887 (textbook) or 418.9829 (reference)
         const float cd = tab[0] * Df;
         return cd - S;
+    } else if constexpr (FUNC == F_REF_ACKLEY) {
+        // -20 expf(-0.2 sqrtf(S / D)) - expf(C / D) + 20 + E with the reference's double
+        // literals -0.2 and E = 2.718282 (SG-EMTF_DE.cu:913)
+        const float o2 = __shfl_xor(s2, 32);
+        const float C = s2 + o2;
+        const float q = S / Df;
+        const float r = sqrtf(q);
+        const float a = (float)(-0.2 * (double)r);
+        const float t1 = -20.0f * exp_f(a);
+        const float c2 = C / Df;
+        const float e2 = exp_f(c2);
+        float u = t1 - e2;
+        u = u + 20.0f;
+        return (float)((double)u + 2.718282);
+    } else if constexpr (FUNC == F_REF_GRIEWANK) {
+        // 1 + S / 4000 - prod (the halves' partial products multiplied once)
+        const float o2 = __shfl_xor(s2, 32);
+        const float P = s2 * o2;
+        const float s4 = S / 4000.0f;
+        const float u = 1.0f + s4;
+        return u - P;
+    } else if constexpr (FUNC == F_REF_WEIERSTRASS) {
+        // sum - D W with the reference's constant W in the task table
+        const float dw = Df * tab[0];
+        return S - dw;
     } else {
         return S;
     }
@@ -274,61 +328,7 @@ __device__ __forceinline__ float objective(const f16v (&acc)[NT], int D, const f
                 }
             }
     }
-    const float o1 = __shfl_xor(s1, 32);
-    const float S = s1 + o1;  // A + B (commutative)
-    const float Df = (float)D;
-    if constexpr (FUNC == F_ACKLEY) {
-        const float o2 = __shfl_xor(s2, 32);
-        const float C = s2 + o2;
-        const float q = S / Df;
-        const float r = sqrtf(q);
-        const float a = -0.2f * r;
-        const float t1 = -20.0f * expm1_f(a);
-        const float c2 = C / Df;
-        const float b = -2.0f * c2;
-        const float t2 = 2.71828175f * expm1_f(b);
-        return t1 - t2;
-    } else if constexpr (FUNC == F_GRIEWANK) {
-        const float o2 = __shfl_xor(s2, 32);
-        const float qA = h ? o2 : s2;
-        const float qB = h ? s2 : o2;
-        const float om = 1.0f - qA;
-        const float tq = qB * om;
-        const float Qv = qA + tq;
-        const float s4 = S / 4000.0f;
-        return s4 + Qv;
-    } else if constexpr (FUNC == F_SCHWEFEL) {
-        // the constant from the task table: 418.982887 (textbook) or 418.9829 (reference)
-        const float cd = tab[0] * Df;
-        return cd - S;
-    } else if constexpr (FUNC == F_REF_ACKLEY) {
-        // -20 expf(-0.2 sqrtf(S / D)) - expf(C / D) + 20 + E with the reference's double
-        // literals -0.2 and E = 2.718282 (SG-EMTF_DE.cu:913)
-        const float o2 = __shfl_xor(s2, 32);
-        const float C = s2 + o2;
-        const float q = S / Df;
-        const float r = sqrtf(q);
-        const float a = (float)(-0.2 * (double)r);
-        const float t1 = -20.0f * exp_f(a);
-        const float c2 = C / Df;
-        const float e2 = exp_f(c2);
-        float u = t1 - e2;
-        u = u + 20.0f;
-        return (float)((double)u + 2.718282);
-    } else if constexpr (FUNC == F_REF_GRIEWANK) {
-        // 1 + S / 4000 - prod (the halves' partial products multiplied once)
-        const float o2 = __shfl_xor(s2, 32);
-        const float P = s2 * o2;
-        const float s4 = S / 4000.0f;
-        const float u = 1.0f + s4;
-        return u - P;
-    } else if constexpr (FUNC == F_REF_WEIERSTRASS) {
-        // sum - D W with the reference's constant W in the task table
-        const float dw = Df * tab[0];
-        return S - dw;
-    } else {
-        return S;
-    }
+    return objective_tail<FUNC>(s1, s2, D, tab, h);
 }
 
 // One 32-row tile (tile jt, accumulators acc) of the objective, in two parts: the row

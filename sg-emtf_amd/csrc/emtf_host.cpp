@@ -38,18 +38,9 @@ extern "C" int emtf_lds_floats_kb(int pop, int kb);
 #define EMTF_DECL_WIDE(nt, al)                                                                             \
     extern "C" int emtf_launch_wide_nt##nt##_a##al(const emtf::EpochArgs* args, const int* order, int n,   \
                                                    int lds_bytes, hipStream_t stream);                     \
-    extern "C" int emtf_launch_wide8_nt##nt##_a##al(const emtf::EpochArgs* args, const int* order, int n,  \
-                                                    int lds_bytes, hipStream_t stream);                    \
     extern "C" int emtf_wide_lds_floats_nt##nt##_a##al(int pop);
 #define EMTF_DECL_WPAIR(nt) EMTF_DECL_WIDE(nt, 0) EMTF_DECL_WIDE(nt, 2)
 EMTF_DECL_WPAIR(2) EMTF_DECL_WPAIR(4) EMTF_DECL_WPAIR(5) EMTF_DECL_WPAIR(6) EMTF_DECL_WPAIR(7) EMTF_DECL_WPAIR(8)
-// the wide kernel with the task's Q image in LDS (NT <= 6, 512 threads)
-#define EMTF_DECL_WIDEQ(nt, al)                                                                            \
-    extern "C" int emtf_launch_wideq_nt##nt##_a##al(const emtf::EpochArgs* args, const int* order, int n,  \
-                                                    int lds_bytes, hipStream_t stream);                    \
-    extern "C" int emtf_wideq_lds_floats_nt##nt##_a##al(int pop);
-#define EMTF_DECL_QPAIR(nt) EMTF_DECL_WIDEQ(nt, 0) EMTF_DECL_WIDEQ(nt, 2)
-EMTF_DECL_QPAIR(2) EMTF_DECL_QPAIR(4) EMTF_DECL_QPAIR(5) EMTF_DECL_QPAIR(6)
 #define EMTF_DECL_POLISH(kb)                                                                                \
     extern "C" int emtf_polish_lds_floats_kb##kb(int pop, int waves, int cpe);                             \
     extern "C" int emtf_launch_polish_kb##kb(const emtf::EpochArgs* args, const int* order, int n, int lds_bytes, \
@@ -79,6 +70,8 @@ extern "C" int emtf_launch_draws(uint64_t seed, int n, const uint32_t* addr, uin
 extern "C" int emtf_launch_elites(const emtf::TaskDev* tasks, int n_tasks, const float* X, const float* fit, int k,
                                   int stride, float* out_x, float* out_f, hipStream_t stream);
 extern "C" int emtf_scratch_resolve(int device, float** out, size_t* capacity);
+extern "C" int emtf_launch_q_images(const emtf::TaskDev* tasks, const int* nt, int n_tasks, const float* Q, float* Qw,
+                                    hipStream_t stream);
 extern "C" int emtf_launch_gen_counter(int32_t* gen, int32_t value, int32_t add, hipStream_t stream);
 extern "C" int emtf_launch_donors(const emtf::TaskDev* tasks, int n_tasks, int g, int32_t* list, hipStream_t stream);
 
@@ -97,29 +90,6 @@ static int pick_nt(int dim) {
     for (int nt : kNT)
         if (32 * nt >= dim) return nt;
     return -1;
-}
-
-// the 512-thread build of the wide kernel (populations of more than four tiles)
-static launch_fn pick_wide8(int nt, bool ga) {
-#define EMTF_CASE(k) \
-    case k: return ga ? emtf_launch_wide8_nt##k##_a2 : emtf_launch_wide8_nt##k##_a0;
-    switch (nt) {
-        EMTF_CASE(2) EMTF_CASE(4) EMTF_CASE(5) EMTF_CASE(6) EMTF_CASE(7) EMTF_CASE(8)
-    }
-#undef EMTF_CASE
-    return nullptr;
-}
-
-static launch_fn pick_wideq(int nt, bool ga, int (**lds)(int)) {
-#define EMTF_CASE(k)                                                                 \
-    case k:                                                                          \
-        *lds = ga ? emtf_wideq_lds_floats_nt##k##_a2 : emtf_wideq_lds_floats_nt##k##_a0; \
-        return ga ? emtf_launch_wideq_nt##k##_a2 : emtf_launch_wideq_nt##k##_a0;
-    switch (nt) {
-        EMTF_CASE(2) EMTF_CASE(4) EMTF_CASE(5) EMTF_CASE(6)
-    }
-#undef EMTF_CASE
-    return nullptr;
 }
 
 static launch_fn pick_wide(int nt, bool ga, int (**lds)(int)) {
@@ -212,7 +182,7 @@ struct Variant {
     const char* name = "";
 };
 
-constexpr int kVariants = 3;
+constexpr int kVariants = 2;
 
 struct Bucket {
     bool wide = false;
@@ -225,7 +195,7 @@ struct Bucket {
     int polish_waves = 0;        // 0: polish off
     int polish_cpe = 1;
     int stream = 0;              // index into the handle's streams (0 = the caller's)
-    Variant v[kVariants];        // [0] primary, [1] [2] alternatives (fn null if none)
+    Variant v[kVariants];        // [0] primary, [1] the wide kernel for an LDS-kernel unit (fn null if none)
     int use = 0;                 // variant launched
     float ms[kVariants] = {};    // calibration times of the variants
 };
@@ -242,7 +212,7 @@ struct emtf_handle {
     float* d_tab = nullptr;
     float* d_mailbox = nullptr;
     float* d_scratch = nullptr;
-    float* d_qw = nullptr;       // padded Q images of the wide tasks
+    float* d_qw = nullptr;       // Q images in operand order of the wide kernel
     int* d_order = nullptr;      // task ids grouped by bucket
     std::vector<Bucket> buckets;
     bool polish = false;
@@ -493,7 +463,7 @@ static int replay_epoch(emtf_handle* h, int g0, int len, hipStream_t s) {
 // appended), so that another process skips the calibration too.
 namespace {
 std::mutex g_tune_mu;
-std::map<std::string, std::string> g_tune;  // batch signature -> per unit "use ms0 ms1 ms2"
+std::map<std::string, std::string> g_tune;  // batch signature -> per unit "use ms0 ms1"
 bool g_tune_file_read = false;
 
 const char* tune_file() {
@@ -512,7 +482,7 @@ static std::string tune_signature(const emtf_handle* h, const std::vector<emtf::
     (void)hipGetDevice(&dev);
     (void)hipGetDeviceProperties(&prop, dev);
     char buf[256];
-    snprintf(buf, sizeof buf, "emtf-tune-1 %s/%d a%d i%d x%d m%d t%d", prop.gcnArchName, prop.multiProcessorCount,
+    snprintf(buf, sizeof buf, "emtf-tune-2 %s/%d a%d i%d x%d m%d t%d", prop.gcnArchName, prop.multiProcessorCount,
              h->p.algo, h->p.n_islands, h->p.exchange_interval, h->p.migrate_interval, h->p.transfer_interval);
     std::string sig = buf;
     for (const Bucket& b : h->buckets) {
@@ -563,7 +533,7 @@ static bool tune_lookup(emtf_handle* h, const std::string& sig) {
     for (size_t k = 0; k < h->buckets.size(); ++k) {
         int u = 0, n = 0;
         float m[kVariants] = {};
-        if (sscanf(q, " %d %f %f %f%n", &u, &m[0], &m[1], &m[2], &n) != 4) return false;
+        if (sscanf(q, " %d %f %f%n", &u, &m[0], &m[1], &n) != 3) return false;
         if (u < 0 || u >= kVariants || !h->buckets[k].v[u].fn) return false;
         use.push_back(u);
         for (int v = 0; v < kVariants; ++v) ms.push_back(m[v]);
@@ -580,7 +550,7 @@ static void tune_store(const emtf_handle* h, const std::string& sig) {
     std::string val;
     char buf[96];
     for (const Bucket& b : h->buckets) {
-        snprintf(buf, sizeof buf, " %d %.6g %.6g %.6g", b.use, b.ms[0], b.ms[1], b.ms[2]);
+        snprintf(buf, sizeof buf, " %d %.6g %.6g", b.use, b.ms[0], b.ms[1]);
         val += buf;
     }
     std::lock_guard<std::mutex> lock(g_tune_mu);
@@ -836,10 +806,8 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
         ++b.count;
     }
 
-    // variants: [0] as chosen above; [1] for an LDS-kernel bucket, the wide kernel for
-    // its largest dimension, for a wide bucket, its 512-thread build; [2] the wide kernel
-    // with Q in LDS where it fits (timed against [0] by the autotuner; not with polish,
-    // whose kernel needs the LDS rows)
+    // variants: [0] as chosen above; [1] for an LDS-kernel bucket, the wide kernel for its
+    // largest dimension (timed against [0] by the autotuner)
     // the persistent schedule runs one LDS-kernel launch unit, without polish or admission
     const bool persist = prm->schedule == EMTF_SCHEDULE_PERSISTENT;
     if (persist) {
@@ -870,42 +838,16 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
                 maxd = std::max(maxd, tasks[t].dim);
                 maxp = std::max(maxp, tasks[t].pop);
             }
-        // the wide kernel with Q in LDS for row geometry nt, when its LDS fits
-        auto add_wideq = [&](int nt) {
-            int (*ql)(int) = nullptr;
-            launch_fn qf = pick_wideq(nt, ga, &ql);
-            if (!qf || 4 * ql(maxp) > kMaxLdsBytes) return;
-            b.v[2].wide = true;
-            b.v[2].geo = nt;
-            b.v[2].fn = qf;
-            b.v[2].lds_bytes = 4 * ql(maxp);
-            b.v[2].name = "wide Q-in-LDS NT";
-        };
-        if (b.wide) {
-            // wide bucket: the 512-thread build when some population spans more than four tiles
-            if (maxp > 128) {
-                b.v[1] = b.v[0];
-                b.v[1].fn = pick_wide8(b.geo, ga);
-                b.v[1].name = "wide x512 NT";
-            }
-            add_wideq(b.geo);
-            continue;
-        }
-        // an LDS-kernel bucket: the wide kernel with Q in LDS always competes; the wide
-        // kernel with Q in L2 only where LDS allows a single workgroup of the LDS kernel
+        if (b.wide) continue;
         const int nt = pick_nt(maxd);
         if (nt <= 0) continue;
-        add_wideq(nt);
         int (*wl)(int) = nullptr;
-        launch_fn wf = 2 * b.lds_bytes > kMaxLdsBytes ? pick_wide(nt, ga, &wl) : nullptr;
-        if (wf) {
-            b.v[1].wide = true;
-            b.v[1].geo = nt;
-            b.v[1].fn = wf;
-            b.v[1].lds_bytes = 4 * wl(maxp);
-            b.v[1].name = "wide NT";
-        }
-        if (b.v[1].fn || b.v[2].fn) alt_nt[k] = nt;
+        b.v[1].wide = true;
+        b.v[1].geo = nt;
+        b.v[1].fn = pick_wide(nt, ga, &wl);
+        b.v[1].lds_bytes = 4 * wl(maxp);
+        b.v[1].name = "wide NT";
+        if (b.v[1].fn) alt_nt[k] = nt;
     }
     for (int t = 0; t < n_tasks; ++t)
         if (alt_nt[bucket_of[t]] > 0) wide_nt[t] = alt_nt[bucket_of[t]];
@@ -943,7 +885,7 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
         if (wide_nt[t] > 0) {
             const int RS = 32 * wide_nt[t] + 4;
             scr = std::max(scr, 2 * (int64_t)popP * RS);  // population rows, trial rows
-            nW += (int64_t)32 * wide_nt[t] * RS;
+            nW += (int64_t)1024 * wide_nt[t] * wide_nt[t];
         }
         nS += scr;
     }
@@ -1080,19 +1022,6 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
         if (d.shift) std::memcpy(V.data() + td.v_off, d.shift, sizeof(float) * d.dim);
         func_table(td.func, d.dim, TB.data() + td.v_off);
     }
-    // wide tasks: Q rows in the kernels' [even | odd] row layout, zero padded to 32 NT rows
-    std::vector<float> QW((size_t)nW, 0.0f);
-    for (int t = 0; t < n_tasks; ++t) {
-        const emtf::TaskDev& td = h->tasks[t];
-        const int nt = wide_nt[t];
-        if (nt < 0) continue;
-        const int RS = 32 * nt + 4, HS = 16 * nt;
-        const float* q = Q.data() + td.q_off;
-        float* w = QW.data() + td.qw_off;
-        for (int j = 0; j < td.dim; ++j)
-            for (int d2 = 0; d2 < td.dim; ++d2) w[(size_t)j * RS + (d2 & 1) * HS + (d2 >> 1)] = q[(size_t)j * td.dim + d2];
-    }
-
     auto alloc = [&](float** ptr, int64_t n) -> int {
         const hipError_t e = hipMalloc((void**)ptr, (size_t)(n > 0 ? n : 1) * sizeof(float));
         if (e != hipSuccess) return fail(EMTF_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
@@ -1134,16 +1063,23 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
     CP(h->d_Q, Q.data(), sizeof(float) * Q.size());
     CP(h->d_shift, V.data(), sizeof(float) * V.size());
     CP(h->d_tab, TB.data(), sizeof(float) * TB.size());
-    if (nW > 0) CP(h->d_qw, QW.data(), sizeof(float) * QW.size());
 #undef CP
-    if (!online && (rc = launch(h, 0, 0, 1, nullptr)) != EMTF_OK) { free_handle(h); return rc; }
+    int* d_nt = nullptr;  // row tiles of the tasks with a Q image; freed after the synchronisation below
+    if (nW > 0) {
+        e = hipMalloc((void**)&d_nt, sizeof(int) * n_tasks);
+        if (e == hipSuccess) e = hipMemcpy(d_nt, wide_nt.data(), sizeof(int) * n_tasks, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = (hipError_t)emtf_launch_q_images(h->d_tasks, d_nt, n_tasks, h->d_Q, h->d_qw, nullptr);
+        if (e != hipSuccess) { (void)hipFree(d_nt); free_handle(h); return fail(EMTF_E_DEVICE, std::string("Q images: ") + hipGetErrorString(e)); }
+    }
+    rc = online ? EMTF_OK : launch(h, 0, 0, 1, nullptr);
     e = hipStreamSynchronize(nullptr);
+    (void)hipFree(d_nt);
+    if (rc != EMTF_OK) { free_handle(h); return rc; }
     if (e != hipSuccess) { free_handle(h); return fail(EMTF_E_DEVICE, std::string("init: ") + hipGetErrorString(e)); }
     if (tune && prm->tune == 0 && (rc = calibrate(h, nX, nF, order)) != EMTF_OK) { free_handle(h); return rc; }
     if (tune && prm->tune >= 2)
         for (Bucket& b : h->buckets) {
-            const int v = prm->tune - 1;
-            b.use = b.v[v].fn ? v : 0;
+            b.use = b.v[1].fn ? 1 : 0;
         }
     *out = h;
     return EMTF_OK;

@@ -31,7 +31,7 @@ struct TaskDev {
     int64_t v_off;    // shift[dim] and per-dimension table[dim]
     int64_t mb_off;   // elite mailbox [transfer_count][dim] inside one mailbox buffer
     int64_t scr_off;  // scratch [pop][row stride] (wide tasks: population rows, then trial rows)
-    int64_t qw_off;   // wide tasks: padded Q image [32 NT][row stride]
+    int64_t qw_off;   // Q image in operand order [4 NT gene blocks][NT row tiles][256]
 };
 
 struct EngineParams {
@@ -58,7 +58,7 @@ struct EpochArgs {
     float* mailbox;
     int64_t mailbox_stride;  // elements per mailbox buffer
     float* scratch;
-    const float* Qw;   // padded Q images of the wide tasks
+    const float* Qw;   // Q images in operand order
     EngineParams p;
     int32_t publish;       // write the task's elites to the mailbox after generation g1
     // Replayed epochs (hipGraph): when set, the epoch starts at *gen_dev instead of g0 and

@@ -143,6 +143,23 @@ __global__ void gen_counter_kernel(int32_t* gen, int32_t value, int32_t add) {
     if (threadIdx.x == 0) gen[0] = add ? gen[0] + value : value;
 }
 
+// Q images in the matrix instructions' operand order: for gene block sb and row tile jt of nt,
+// float 256 (sb nt + jt) + 4 l + e is Q[32 jt + (l & 31)][2 (4 sb + e) + (l >> 5)], zero past the
+// dimension.  One workgroup per task; nt: row tiles of every task, no image where not positive.
+__global__ __launch_bounds__(256) void q_image_kernel(const TaskDev* __restrict__ tasks, const int* __restrict__ nt,
+                                                      const float* __restrict__ Q, float* __restrict__ Qw) {
+    const int NT = nt[blockIdx.x];
+    if (NT <= 0) return;
+    const TaskDev td = tasks[blockIdx.x];
+    const int D = td.dim, e = threadIdx.x & 3, l = threadIdx.x >> 2;
+    for (int b = 0; b < 4 * NT * NT; ++b) {
+        const int sb = b / NT, jt = b - sb * NT;
+        const int j = 32 * jt + (l & 31), d = 2 * (4 * sb + e) + (l >> 5);
+        const bool in = j < D && d < D;
+        Qw[td.qw_off + 256 * b + threadIdx.x] = in ? Q[td.q_off + (int64_t)j * D + d] : 0.0f;
+    }
+}
+
 // n int32 values set to v (the persistent schedule's counters; a kernel, not a memset, so
 // the call can sit in a captured graph).
 __global__ void fill_i32_kernel(int32_t* p, int n, int32_t v) {
@@ -155,6 +172,12 @@ extern "C" int emtf_launch_fill_i32(int32_t* p, int n, int32_t value, hipStream_
     if (n <= 0) return 0;
     const int blocks = (n + 255) / 256 < 1024 ? (n + 255) / 256 : 1024;
     hipLaunchKernelGGL(emtf::fill_i32_kernel, dim3(blocks), dim3(256), 0, stream, p, n, value);
+    return (int)hipGetLastError();
+}
+
+extern "C" int emtf_launch_q_images(const emtf::TaskDev* tasks, const int* nt, int n_tasks, const float* Q, float* Qw,
+                                    hipStream_t stream) {
+    hipLaunchKernelGGL(emtf::q_image_kernel, dim3(n_tasks), dim3(256), 0, stream, tasks, nt, Q, Qw);
     return (int)hipGetLastError();
 }
 

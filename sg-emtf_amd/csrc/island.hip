@@ -51,6 +51,16 @@ struct Shape {
 template <int KB>
 constexpr int kSkipBlock = KB == 4 ? 3 : (KB == 7 ? 5 : (KB == 12 ? 10 : (KB == 16 ? 14 : 0)));
 
+// Q in the matrix instructions' operand order (an image built on the device when a batch is
+// created): 256 floats per gene block and row tile, lane l's four the genes of the block in half
+// l >> 5 of row 32 jt + (l & 31), zero past the dimension.  A wave's read is 1 KB of consecutive
+// bytes -- from L2 where a row-major matrix costs 64 lines of 16 bytes each, from LDS without a
+// bank conflict or the rows' padding.
+__device__ __forceinline__ float4 q_op(const float* q, int nt, int sb, int jt) {
+    const float* p = q + 256 * (sb * nt + jt);
+    return make_float4(p[0], p[1], p[2], p[3]);
+}
+
 struct Geo {
     int D, Dh, pop, popP, ntiles, m;
     FastMod modD, modM;  // jrand = w mod D, island-local index = w mod m
@@ -1462,26 +1472,35 @@ __global__ __launch_bounds__(kThreads) EMTF_OCCUPANCY void island_persistent_ker
 
 #if defined(EMTF_WIDE_NT)
 // ---------------------------------------------------------------------------
-// Wide tasks: dimensions up to 32 NT whose rows (or whose population) do not fit
-// LDS.  The population rows X, the trial rows T and the task's padded Q image
-// live in global memory (a task's working set stays L2-resident while its
-// workgroup runs); LDS keeps o, the per-dimension table and the fitness and
-// rank arrays.  Trial genes are formed block by block and fed straight into the
-// MFMA k-loop as the B operand, and stored to T for the selection copy, so no
-// lane holds a whole row in registers.  Rows use the LDS path's [even | odd]
-// layout with HS = 16 NT; the gene order of every fma chain is the LDS path's,
-// with the padded k-steps past the dimension skipped (they would add +0).
+// Wide tasks: dimensions up to 32 NT, any population.  The population's rows live in global
+// memory (a task's working set stays L2-resident while its workgroup runs), two rows per
+// individual: the individual and its trial, which change roles when the trial is accepted
+// (L.off[i], the individual's row).  LDS keeps the task's Q image where it fits (QL; else it
+// is read from L2), o, the per-dimension table and the per-individual arrays.  A generation
+// of the eight waves has three phases:
+//   mates   one thread per individual draws its mates and leaves their row offsets in LDS;
+//   trials  one thread per (individual, parity half, octet of genes): a Philox block's eight
+//           crossover draws, 32 contiguous bytes of each parent row -- with the matrix
+//           instructions' mapping (an individual per column) a load touched 64 rows for 16
+//           bytes of each, and the rows went through L1 eight times over;
+//   fitness z = Q w by v_mfma_f32_32x32x2_f32 over the trial rows, then the objective.  A wave
+//           per tile of 32 individuals where there are five tiles or more, else the tile's row
+//           tiles are dealt to 2, 4 or 8 waves: each computes the terms of its rows, and the
+//           sums run through the waves in row order (so the bits are those of one wave).
+// What bounds it: for large populations the fitness phase's MFMA (32 NT cycles a gene and tile)
+// and then the trials' row traffic (256 tasks of D = 150, pop 256 read and write 240 MB a
+// generation, 5 TB/s through L2 and the last-level cache), for small ones barriers and latencies.
+// An epoch of 20 generations of 256 sphere tasks, against a kernel that formed the trials in the
+// matrix instructions' mapping (its fastest build): D = 150, pop 32 / 128 / 256 0.495 / 0.661 /
+// 1.365 to 0.257 / 0.609 / 1.017 ms; D = 180, pop 128 / 256 0.828 / 1.701 to 0.717 / 1.321; D = 200
+// (Q from L2) 1.819 / 4.087 to 1.004 / 1.700.  Rows use the LDS path's [even | odd]
+// layout with HS = 16 NT; the gene order of every fma chain is the LDS path's, with the padded
+// k-steps past the dimension skipped (they would add +0).
 // ---------------------------------------------------------------------------
+constexpr int kWideThreads = 512, kWideWaves = kWideThreads / 64;
+
 template <int NT>
 using WShape = Shape<4 * NT>;
-
-// Q operands of gene block sb: rows 32 jt + col of the lane's half
-template <int NT>
-__device__ __forceinline__ void load_q(float4 (&q)[NT], const float* qrow, int sb) {
-    using S = WShape<NT>;
-#pragma unroll
-    for (int jt = 0; jt < NT; ++jt) q[jt] = lds4(qrow + 32 * jt * S::RS + 4 * sb);
-}
 
 // acc[jt] += Q rows (32 jt + col) x (4 genes of one block of the lane's half)
 template <int NT>
@@ -1494,9 +1513,10 @@ __device__ __forceinline__ void mfma_q(f16v (&acc)[NT], const float4 (&q)[NT], c
 }
 
 template <int NT>
-__device__ __forceinline__ void mfma_block(f16v (&acc)[NT], const float* qrow, const float4& w4, int sb) {
+__device__ __forceinline__ void mfma_block(f16v (&acc)[NT], const float* ql, const float4& w4, int sb) {
     float4 q[NT];
-    load_q<NT>(q, qrow, sb);
+#pragma unroll
+    for (int jt = 0; jt < NT; ++jt) q[jt] = q_op(ql, NT, sb, jt);
     mfma_q<NT>(acc, q, w4);
 }
 
@@ -1518,132 +1538,257 @@ __device__ __forceinline__ float wide_eval_row(const float* row_h, const Geo& g,
     using S = WShape<NT>;
     f16v acc[NT];
     zero_acc<NT>(acc);
-    const float* qrow = L.Q + col * S::RS + h * S::HS;
+    const float* ql = L.Q + 4 * (32 * h + col);
     const float* orow = L.o + h * S::HS;
-    for (int sb = 0; sb < nsb; ++sb) mfma_block<NT>(acc, qrow, sub4(lds4(row_h + 4 * sb), lds4(orow + 4 * sb)), sb);
+    for (int sb = 0; sb < nsb; ++sb) mfma_block<NT>(acc, ql, sub4(lds4(row_h + 4 * sb), lds4(orow + 4 * sb)), sb);
     return objective<NT, FUNC, true>(acc, g.D, L.tab, h);
 }
 
-template <int NT, int FUNC, int ALGO, int WT, bool QL>
-__device__ __forceinline__ void wide_generation(const EpochArgs& a, const TaskDev& td, const Geo& g, const Lds& L,
-                                                float* T, const Rng& rng, int gen, int tid, int nsb) {
+// LDS of a wide task behind the Q image (QL).  `shared` holds the mates while trials are formed,
+// the split sums while fitness is computed, and the scratch, rank and flag arrays between.
+struct WideLds {
+    int* off;    // popP: the individual's row, in floats from the first row
+    int4* mate;  // popP: row offsets of the three mates (GA: two) and of the individual
+    int* jr;     // popP: jrand
+    float* ps;   // 4 tiles x 128: running sums s1 | s2 per lane
+    float* pz;   // 8 waves x 32: Rosenbrock, row 0 of the wave's first row tile
+};
+
+__host__ __device__ inline int wide_lds_floats(int nt, int pop, bool ql) {
+    const int RS = 32 * nt + 4, popP = (pop + 31) & ~31, sh = 5 * popP > 1280 ? 5 * popP : 1280;
+    return (ql ? 1024 * nt * nt : 0) + RS + 32 * nt + 2 * popP + sh;
+}
+
+// Mates of every individual as row offsets.
+template <int ALGO>
+__device__ __forceinline__ void wide_mates(const EpochArgs& a, const Geo& g, const WideLds& W, const Rng& rng, int gen,
+                                           int tid) {
+    for (int i = tid; i < g.pop; i += kWideThreads) {
+        const int il = (int)g.modM.mod((uint32_t)i), base = i - il;
+        int4 m;
+        if constexpr (ALGO == A_GA_SBX_PM) {
+            const U4 mb = rng.block((uint32_t)gen, P_GA_MATE, (uint32_t)(i & ~1), 0u, 0u);
+            m.x = W.off[base + (int)g.modM.mod(pick(mb, (uint32_t)(il & 1)))];
+            m.y = W.off[base + (int)g.modM.mod(pick(mb, (uint32_t)((il & 1) ^ 1)))];
+            m.z = 0;
+        } else {
+            const DeMates mt = de_mates(a, g, rng, gen, i);
+            m.x = W.off[a.p.algo == A_DE_RAND_1_BIN ? base + mt.r1 : i];
+            m.y = W.off[base + mt.r2];
+            m.z = W.off[base + mt.r3];
+            W.jr[i] = mt.jrand;
+        }
+        m.w = W.off[i];
+        W.mate[i] = m;
+    }
+}
+
+// Trial rows: unit e = (individual i, half h, octet o), U units per individual; i0, r0: the
+// thread's first unit, di, dr: its step.
+template <int NT, int ALGO>
+__device__ __forceinline__ void wide_trials(const EpochArgs& a, const TaskDev& td, const Geo& g, float* X,
+                                            const WideLds& W, const Rng& rng, int gen, int i0, int r0, int U) {
     using S = WShape<NT>;
     constexpr int RS = S::RS, HS = S::HS;
-    const int wave = tid >> 6, lane = tid & 63, col = lane & 31;
-    for (int it = wave; it < g.ntiles; it += WT / 64) {
-        // the lane's half index is made opaque per tile (masks derived from it are not
-        // hoisted out of the generation loop into spilled scalar registers)
-        int h = lane >> 5;
-        asm volatile("" : "+v"(h));
-        const float* qrow = L.Q + col * RS + h * HS;
-        const float* orow = L.o + h * HS;
-        const int i = it * 32 + col;
-        const bool valid = i < g.pop;
-        const int ie = valid ? i : 0;
-        const int il = (int)g.modM.mod((uint32_t)ie), base = ie - il;
-        float* trow = T + (int64_t)i * RS + h * HS;
-        f16v acc[NT];
-        zero_acc<NT>(acc);
+    const int noct = U >> 1, di = kWideThreads / U, dr = kWideThreads - di * U;
+    int i = i0, r = r0;
+    DeConst dc{};
+    GaConst gc{};
+    if constexpr (ALGO == A_GA_SBX_PM) gc = ga_const(a, td);
+    else dc = de_const(a, td);
+    while (i < g.pop) {
+        const int h = r >= noct ? 1 : 0, o = r - (h ? noct : 0), c = h * HS + 8 * o;
+        const int4 m = W.mate[i];
+        float* dst = X + (2 * i + g.popP) * RS - m.w + c;  // the individual's other row
+        const float *pa = X + m.x + c, *pb = X + m.y + c;
+        float4 out[2];
         if constexpr (ALGO == A_GA_SBX_PM) {
-            const U4 mb = rng.block((uint32_t)gen, P_GA_MATE, (uint32_t)(ie & ~1), 0u, 0u);
-            const int ra = (int)g.modM.mod(pick(mb, (uint32_t)(il & 1)));
-            const int rb = (int)g.modM.mod(pick(mb, (uint32_t)((il & 1) ^ 1)));
-            const float* xa = L.X + (int64_t)(base + ra) * RS + h * HS;
-            const float* xb = L.X + (int64_t)(base + rb) * RS + h * HS;
-            const GaConst c0 = ga_const(a, td);
-            const bool odd = (il & 1) != 0;
-            float4 na = lds4(xa), nb = lds4(xb);
-            float4 nq[NT];
-            if constexpr (!QL) load_q<NT>(nq, qrow, 0);
-            for (int sb = 0; sb < nsb; ++sb) {
-                const float4 va = na, vb = nb;
-                float4 q[NT];
-                if constexpr (QL) {
-                    load_q<NT>(q, qrow, sb);
-                } else {
-#pragma unroll
-                    for (int jt = 0; jt < NT; ++jt) q[jt] = nq[jt];
-                }
-                if (sb + 1 < nsb) {
-                    na = lds4(xa + 4 * (sb + 1));
-                    nb = lds4(xb + 4 * (sb + 1));
-                    if constexpr (!QL) load_q<NT>(nq, qrow, sb + 1);
-                }
+#pragma unroll 1
+            for (int b = 0; b < 2; ++b) {
                 float t[4];
-                ga_block(t, va, vb, rng, gen, ie, sb, h, odd, g.D, c0);
-                const float4 t4 = make_float4(t[0], t[1], t[2], t[3]);
-                *reinterpret_cast<float4*>(trow + 4 * sb) = t4;
-                mfma_q<NT>(acc, q, sub4(t4, lds4(orow + 4 * sb)));
+                ga_block(t, lds4(pa + 4 * b), lds4(pb + 4 * b), rng, gen, i, 2 * o + b, h, (i & 1) != 0, g.D, gc);
+                *reinterpret_cast<float4*>(dst + 4 * b) = make_float4(t[0], t[1], t[2], t[3]);
             }
         } else {
-            const bool rand1 = (a.p.algo == A_DE_RAND_1_BIN);
-            const DeMates mt = de_mates(a, g, rng, gen, ie);
-            const float* xb = L.X + (int64_t)(base + (rand1 ? mt.r1 : il)) * RS + h * HS;
-            const float* x2 = L.X + (int64_t)(base + mt.r2) * RS + h * HS;
-            const float* x3 = L.X + (int64_t)(base + mt.r3) * RS + h * HS;
-            const float* xi = L.X + (int64_t)ie * RS + h * HS;
-            // global-memory operands of block sb + 1 are loaded while block sb computes
-            DeConst dc = de_const(a, td);
-            dc.jr = mt.jrand - h;
-            U4 cb{0u, 0u, 0u, 0u};
-            float4 nb = lds4(xb), n2 = lds4(x2), n3 = lds4(x3), ni = lds4(xi);
-            float4 nq[NT];
-            if constexpr (!QL) load_q<NT>(nq, qrow, 0);
-            for (int sb = 0; sb < nsb; ++sb) {
-                const float4 vb = nb, v2 = n2, v3 = n3, vi = ni;
-                float4 q[NT];
-                if constexpr (QL) {
-                    load_q<NT>(q, qrow, sb);
-                } else {
+            const float *pc = X + m.z + c, *pi = X + m.w + c;
+            float4 va[2], vb[2], vc[2], vi[2];
 #pragma unroll
-                    for (int jt = 0; jt < NT; ++jt) q[jt] = nq[jt];
-                }
-                if (sb + 1 < nsb) {
-                    const int o = 4 * (sb + 1);
-                    nb = lds4(xb + o);
-                    n2 = lds4(x2 + o);
-                    n3 = lds4(x3 + o);
-                    ni = lds4(xi + o);
-                    if constexpr (!QL) load_q<NT>(nq, qrow, sb + 1);
-                }
-                if ((sb & 1) == 0) cb = rng.block((uint32_t)gen, P_DE_CR, (uint32_t)ie, (uint32_t)h, (uint32_t)(sb >> 1));
+            for (int b = 0; b < 2; ++b) {
+                va[b] = lds4(pa + 4 * b);
+                vb[b] = lds4(pb + 4 * b);
+                vc[b] = lds4(pc + 4 * b);
+                vi[b] = lds4(pi + 4 * b);
+            }
+            const U4 cb = rng.block((uint32_t)gen, P_DE_CR, (uint32_t)i, (uint32_t)h, (uint32_t)o);
+            dc.jr = W.jr[i] - h - 16 * o;
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
                 float t[4];
-                de_block(t, vb, v2, v3, vi, cb, sb, dc);
-                const float4 t4 = make_float4(t[0], t[1], t[2], t[3]);
-                *reinterpret_cast<float4*>(trow + 4 * sb) = t4;
-                mfma_q<NT>(acc, q, sub4(t4, lds4(orow + 4 * sb)));
+                de_block(t, va[b], vb[b], vc[b], vi[b], cb, b, dc);
+                out[b] = make_float4(t[0], t[1], t[2], t[3]);
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) *reinterpret_cast<float4*>(dst + 4 * b) = out[b];
+        }
+        i += di;
+        r += dr;
+        if (r >= U) {
+            r -= U;
+            ++i;
+        }
+    }
+}
+
+// z rows of R row tiles from jt0 of the lane's trial row (its parity half at trow, global
+// memory): four gene blocks (64 bytes) of the row loaded at a time, the next four while these
+// are multiplied.  Row tiles past the last repeat it (their z is not used).
+template <int NT, int R, bool QL>
+__device__ __forceinline__ void wide_z(f16v (&acc)[R], const float* trow, const float* Q, int jt0, const float* orow,
+                                       int col, int h, int nsb) {
+    zero_acc<R>(acc);
+    const float* qt[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) qt[r] = Q + 4 * (32 * h + col) + 256 * (jt0 + r < NT ? jt0 + r : NT - 1);
+    float4 nb[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) nb[k] = lds4(trow + 4 * k);
+    float4 q[R];
+    if constexpr (!QL) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) q[r] = q_op(qt[r], NT, 0, 0);
+    }
+#pragma unroll 1
+    for (int s0 = 0; s0 < nsb; s0 += 4) {
+        float4 b[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) b[k] = nb[k];
+        if (s0 + 4 < nsb) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) nb[k] = lds4(trow + 4 * (s0 + 4 + k));
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int sb = s0 + k;
+            if (k > 0 && sb >= nsb) break;
+            const float4 w = sub4(b[k], lds4(orow + 4 * sb));
+            if constexpr (QL) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) q[r] = q_op(qt[r], NT, sb, 0);
+                mfma_q<R>(acc, q, w);
+            } else {
+                // Q from L2: a row tile's four steps, then its operands of the next block
+                // into the same registers
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[r] = __builtin_amdgcn_mfma_f32_32x32x2f32(f4(q[r], e), f4(w, e), acc[r], 0, 0, 0);
+                    if (sb + 1 < nsb) q[r] = q_op(qt[r], NT, sb + 1, 0);
+                }
             }
         }
+    }
+}
+
+// The individual's trial replaces it when its fitness is no worse.
+__device__ __forceinline__ void wide_select(const Geo& g, const Lds& L, const WideLds& W, int RS, int i, int h, float f) {
+    if (i < g.pop && h == 0 && L.fit[i] >= f) {
+        L.fit[i] = f;
+        W.off[i] = (2 * i + g.popP) * RS - W.off[i];
+    }
+}
+
+// Fitness of the trials, a wave per tile.
+template <int NT, int FUNC, bool QL>
+__device__ __forceinline__ void wide_fitness(const Geo& g, const Lds& L, const WideLds& W, int wave, int col, int h, int nsb) {
+    using S = WShape<NT>;
+    for (int it = wave; it < g.ntiles; it += kWideWaves) {
+        const int i = it * 32 + col;
+        const float* trow = L.X + (2 * i + g.popP) * S::RS - W.off[i] + h * S::HS;
+        f16v acc[NT];
+        wide_z<NT, NT, QL>(acc, trow, L.Q, 0, L.o + h * S::HS, col, h, nsb);
         const float f = objective<NT, FUNC, true>(acc, g.D, L.tab, h);
-        const bool accept = valid && (L.fit[i] >= f);
-        if (valid && h == 0) {
-            L.aux[i] = accept ? 1 : 0;
-            L.ftmp[i] = f;
+        wide_select(g, L, W, S::RS, i, h, f);
+    }
+}
+
+// Fitness of the trials of at most four tiles, each tile's row tiles dealt R at a time to
+// kWideWaves / ... waves (SP waves per tile, wave = SP tile + group).  Every wave takes part in
+// the barriers.
+template <int NT, int FUNC, bool QL, int R, int SP>
+__device__ __forceinline__ void wide_fitness_split(const Geo& g, const Lds& L, const WideLds& W, int wave, int lane, int col,
+                                                   int h, int nsb) {
+    using S = WShape<NT>;
+    constexpr int NG = (NT + R - 1) / R;  // groups of row tiles
+    static_assert(NG <= SP && R * SP >= NT, "every row tile has a wave");
+    const int it = wave / SP, grp = wave % SP;
+    const bool active = it < g.ntiles && grp < NG;
+    const int i = (it < g.ntiles ? it : 0) * 32 + col, jt0 = grp * R;
+    f16v acc[R];
+    float v1[R][16], v2[R][16];
+    if (active) {
+        const float* trow = L.X + (2 * i + g.popP) * S::RS - W.off[i] + h * S::HS;
+        wide_z<NT, R, QL>(acc, trow, L.Q, jt0, L.o + h * S::HS, col, h, nsb);
+        if (FUNC == F_ROSENBROCK && h == 0) W.pz[32 * wave + col] = acc[0][0];
+    }
+    if constexpr (FUNC == F_ROSENBROCK) __syncthreads();
+    if (active) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float zn0 = 0.0f;  // row 32 (jt + 1) of z
+            if constexpr (FUNC == F_ROSENBROCK) {
+                if (r + 1 < R) zn0 = __shfl_xor(acc[r + 1 < R ? r + 1 : r][0], 32);
+                else if (grp + 1 < NG) zn0 = W.pz[32 * (wave + 1) + col];
+            }
+            if (jt0 + r < NT) tile_vals<FUNC>(acc[r], jt0 + r, g.D, L.tab, h, zn0, v1[r], v2[r]);
         }
+    }
+    for (int st = 0; st < NG; ++st) {
+        if (active && grp == st) {
+            float s1, s2;
+            sums_start<FUNC>(s1, s2);
+            if (st > 0) {
+                s1 = W.ps[128 * it + lane];
+                s2 = W.ps[128 * it + 64 + lane];
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (jt0 + r < NT) tile_sums<FUNC>(v1[r], v2[r], jt0 + r, g.D, h, s1, s2);
+            if (st + 1 < NG) {
+                W.ps[128 * it + lane] = s1;
+                W.ps[128 * it + 64 + lane] = s2;
+            } else {
+                const float f = objective_tail<FUNC>(s1, s2, g.D, L.tab, h);
+                wide_select(g, L, W, S::RS, i, h, f);
+            }
+        }
+        if (st + 1 < NG) __syncthreads();
+    }
+}
+
+// Every individual's row back in the first set of rows (before phases that move rows).
+template <int NT>
+__device__ __forceinline__ void wide_gather(const Geo& g, const Lds& L, const WideLds& W, int tid) {
+    constexpr int RS = WShape<NT>::RS;
+    for (int e = tid; e < g.pop * (RS / 4); e += kWideThreads) {
+        const int i = e / (RS / 4), c = 4 * (e - i * (RS / 4));
+        if (W.off[i] != i * RS) *reinterpret_cast<float4*>(L.X + i * RS + c) = lds4(L.X + W.off[i] + c);
     }
     __syncthreads();
-    for (int e = tid; e < g.pop * 2 * nsb; e += WT) {
-        const int row = e / (2 * nsb), blk = e - row * (2 * nsb);
-        if (L.aux[row]) {
-            const int c = (blk < nsb) ? 4 * blk : HS + 4 * (blk - nsb);
-            *reinterpret_cast<float4*>(L.X + (int64_t)row * RS + c) = lds4(T + (int64_t)row * RS + c);
-        }
-    }
-    for (int i = tid; i < g.pop; i += WT)
-        if (L.aux[i]) L.fit[i] = L.ftmp[i];
+    for (int i = tid; i < g.popP; i += kWideThreads) W.off[i] = i * RS;
     __syncthreads();
 }
 
 // Inter-task transfer for wide tasks: candidates streamed into the k-loop and
 // staged in T (row j for candidate j), accepted ones copied to their target row.
-template <int NT, int FUNC, int WT>
+template <int NT, int FUNC>
 __device__ __forceinline__ void wide_transfer_in(const EpochArgs& a, const TaskDev& td, const Geo& g, const Lds& L,
                                                  float* T, const Rng& rng, int tid, int nsb) {
     using S = WShape<NT>;
     constexpr int RS = S::RS, HS = S::HS;
     const int k = a.p.transfer_count, TI = a.p.transfer_interval, g0 = a.g0 - td.gen_base;
     const int wave = tid >> 6, lane = tid & 63, col = lane & 31, h = lane >> 5;
-    rank_islands<WT>(L, g.pop, g.pop, tid);
+    rank_islands<kWideThreads>(L, g.pop, g.pop, tid);
     __syncthreads();
     const uint32_t wd = rng.word((uint32_t)g0, P_MIG, 0u, 0u, 0u);
     const int dn = pick_donor(a, (int)rng.task, wd);
@@ -1651,10 +1796,10 @@ __device__ __forceinline__ void wide_transfer_in(const EpochArgs& a, const TaskD
     const float* mb = a.mailbox + (int64_t)((a.g0 / TI) & 1) * a.mailbox_stride + dd.mb_off;
     const bool same_box = (dd.lo == td.lo && dd.hi == td.hi);
     const float rng_s = td.hi - td.lo, rng_d = dd.hi - dd.lo;
-    const float* qrow = L.Q + col * RS + h * HS;
+    const float* ql = L.Q + 4 * (32 * h + col);
     const float* orow = L.o + h * HS;
     const int ntc = (k + 31) / 32;
-    for (int ct = wave; ct < ntc; ct += WT / 64) {
+    for (int ct = wave; ct < ntc; ct += kWideThreads / 64) {
         const int j = ct * 32 + col;
         const bool valid = j < k;
         const int je = valid ? j : 0;
@@ -1688,7 +1833,7 @@ __device__ __forceinline__ void wide_transfer_in(const EpochArgs& a, const TaskD
             }
             const float4 c4 = make_float4(c[0], c[1], c[2], c[3]);
             *reinterpret_cast<float4*>(crow + 4 * sb) = c4;
-            mfma_block<NT>(acc, qrow, sub4(c4, lds4(orow + 4 * sb)), sb);
+            mfma_block<NT>(acc, ql, sub4(c4, lds4(orow + 4 * sb)), sb);
         }
         const float f = objective<NT, FUNC, true>(acc, g.D, L.tab, h);
         if (valid) {
@@ -1703,12 +1848,12 @@ __device__ __forceinline__ void wide_transfer_in(const EpochArgs& a, const TaskD
     __syncthreads();
 }
 
-// QL: the task's Q image is staged in LDS (the workgroup's first 32 NT x RS floats) and
-// the MFMA A operands come from there instead of L2.
-template <int NT, int FUNC, int ALGO, int WT, bool QL>
+// QL: the task's Q image is staged in LDS (the workgroup's first 1024 NT^2 floats) and the
+// MFMA A operands come from there instead of L2.
+template <int NT, int FUNC, int ALGO, bool QL>
 __device__ __forceinline__ void wide_body(const EpochArgs& a, float* smem, const int task, const TaskDev& td) {
     using S = WShape<NT>;
-    constexpr int RS = S::RS, HS = S::HS;
+    constexpr int RS = S::RS, HS = S::HS, WT = kWideThreads;
     const int tid = threadIdx.x;
     Geo g;
     g.D = td.dim;
@@ -1726,10 +1871,10 @@ __device__ __forceinline__ void wide_body(const EpochArgs& a, float* smem, const
     float* base = smem;
     if constexpr (QL) {
         L.Q = smem;
-        base = smem + 32 * NT * RS;
+        base = smem + 1024 * NT * NT;
         // eight 16-byte loads in flight per thread
         const float4* qg = reinterpret_cast<const float4*>(a.Qw + td.qw_off);
-        constexpr int n4 = 32 * NT * RS / 4;
+        constexpr int n4 = 256 * NT * NT;
         for (int e0 = tid; e0 < n4; e0 += 8 * WT) {
             float4 v[8];
 #pragma unroll
@@ -1749,13 +1894,21 @@ __device__ __forceinline__ void wide_body(const EpochArgs& a, float* smem, const
     L.o = base;
     L.tab = L.o + RS;
     L.fit = L.tab + 32 * NT;
-    L.ftmp = L.fit + g.popP;
-    L.ord = reinterpret_cast<int*>(L.ftmp + g.popP);
+    WideLds W;
+    W.off = reinterpret_cast<int*>(L.fit + g.popP);
+    float* sh = reinterpret_cast<float*>(W.off + g.popP);
+    W.mate = reinterpret_cast<int4*>(sh);
+    W.jr = reinterpret_cast<int*>(sh + 4 * g.popP);
+    W.ps = sh;
+    W.pz = sh + 512;
+    L.ftmp = sh;
+    L.ord = reinterpret_cast<int*>(sh + g.popP);
     L.aux = L.ord + g.popP;
     const Rng rng{a.p.seed_lo, a.p.seed_hi, (uint32_t)task};
-    const int lane = tid & 63, col = lane & 31, h = lane >> 5, wave = tid >> 6;
+    const int lane = tid & 63, col = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     for (int e = tid; e < RS + 32 * NT; e += WT) base[e] = 0.0f;
+    for (int i = tid; i < g.popP; i += WT) W.off[i] = i * RS;
     __syncthreads();
     for (int d = tid; d < g.D; d += WT) {
         L.o[(d & 1) * HS + (d >> 1)] = a.shift[td.v_off + d];
@@ -1809,21 +1962,39 @@ __device__ __forceinline__ void wide_body(const EpochArgs& a, float* smem, const
     }
 
     const int TI = a.p.transfer_interval;
-    if (transfer_now(a, td)) wide_transfer_in<NT, FUNC, WT>(a, td, g, L, T, rng, tid, nsb);
+    if (transfer_now(a, td)) wide_transfer_in<NT, FUNC>(a, td, g, L, T, rng, tid, nsb);
 
+    const int U = 2 * ((g.Dh + 7) >> 3);  // trial units per individual
+    const int ti0 = tid / U, tr0 = tid - ti0 * U;
     const bool islands = a.p.n_islands > 1;
     for (int gen = a.g0 - td.gen_base + 1; gen <= a.g1 - td.gen_base; ++gen) {
-        if (islands && a.p.exchange_interval > 0 && gen % a.p.exchange_interval == 0)
+        if (islands && a.p.exchange_interval > 0 && gen % a.p.exchange_interval == 0) {
+            wide_gather<NT>(g, L, W, tid);
             island_exchange<4 * NT, WT>(a, g, L, T, rng, gen, tid);
-        wide_generation<NT, FUNC, ALGO, WT, QL>(a, td, g, L, T, rng, gen, tid, nsb);
-        if (islands && a.p.migrate_interval > 0 && a.p.migrate_count > 0 && gen % a.p.migrate_interval == 0)
+        }
+        wide_mates<ALGO>(a, g, W, rng, gen, tid);
+        __syncthreads();
+        wide_trials<NT, ALGO>(a, td, g, L.X, W, rng, gen, ti0, tr0, U);
+        __syncthreads();
+        // the lane's half index is made opaque (masks derived from it are not hoisted out of
+        // the generation loop into spilled scalar registers)
+        int hh = h;
+        asm volatile("" : "+v"(hh));
+        if (g.ntiles > 4) wide_fitness<NT, FUNC, QL>(g, L, W, wave, col, hh, nsb);
+        else if (g.ntiles > 2) wide_fitness_split<NT, FUNC, QL, (NT + 1) / 2, 2>(g, L, W, wave, lane, col, hh, nsb);
+        else if (g.ntiles > 1) wide_fitness_split<NT, FUNC, QL, (NT + 3) / 4, 4>(g, L, W, wave, lane, col, hh, nsb);
+        else wide_fitness_split<NT, FUNC, QL, 1, 8>(g, L, W, wave, lane, col, hh, nsb);
+        __syncthreads();
+        if (islands && a.p.migrate_interval > 0 && a.p.migrate_count > 0 && gen % a.p.migrate_interval == 0) {
+            wide_gather<NT>(g, L, W, tid);
             island_migration<4 * NT, WT>(a, g, L, tid);
+        }
     }
 
     float* Xo = a.X + td.x_off;
     for (int e = tid; e < g.pop * g.D; e += WT) {
         const int i = e / g.D, d = e - i * g.D;
-        Xo[e] = L.X[(int64_t)i * RS + (d & 1) * HS + (d >> 1)];
+        Xo[e] = L.X[W.off[i] + (d & 1) * HS + (d >> 1)];
     }
     for (int i = tid; i < g.pop; i += WT) a.fit[td.fit_off + i] = L.fit[i];
     if (a.publish) {
@@ -1834,44 +2005,38 @@ __device__ __forceinline__ void wide_body(const EpochArgs& a, float* smem, const
         float* mb = a.mailbox + (int64_t)((a.g1 / TI) & 1) * a.mailbox_stride + td.mb_off;
         for (int e = tid; e < k * g.D; e += WT) {
             const int r = e / g.D, d = e - r * g.D;
-            mb[e] = L.X[(int64_t)L.ord[r] * RS + (d & 1) * HS + (d >> 1)];
+            mb[e] = L.X[W.off[L.ord[r]] + (d & 1) * HS + (d >> 1)];
         }
     }
 }
 
-// Two waves per SIMD: a wave's MFMA k-loop then overlaps another wave's trial
-// formation and objective epilogue (one wave per SIMD leaves the MFMA pipe idle
-// through both).  Workgroups of 256 threads (two per CU) or, for populations of
-// more than four 32-row tiles, 512 threads (one per CU, half the tiles per wave).
-// WPE: the waves per SIMD the register allocation targets (1: no target)
-constexpr int kWideWpe = EMTF_WIDE_NT <= 6 ? 2 : 1;
-
-template <int NT, int ALGO, int WT, bool QL, int WPE>
-__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(WPE))) void wide_epoch_kernel(
+// Two waves per SIMD: one workgroup of eight waves a CU at the largest Q images, and at least
+// that at the others.
+template <int NT, int ALGO, bool QL>
+__global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(2))) void wide_epoch_kernel(
     EpochArgs a, const int* __restrict__ order) {
-    extern __shared__ float smem[];
+    extern __shared__ __align__(16) float smem[];
     rebase_epoch(a);
     const int task = order[blockIdx.x];
     const TaskDev td = a.tasks[task];
     if (!runs_epoch(a, td)) return;
     switch (td.func) {
-    case F_SPHERE: wide_body<NT, F_SPHERE, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_ROSENBROCK: wide_body<NT, F_ROSENBROCK, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_ACKLEY: wide_body<NT, F_ACKLEY, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_RASTRIGIN: wide_body<NT, F_RASTRIGIN, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_GRIEWANK: wide_body<NT, F_GRIEWANK, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_WEIERSTRASS: wide_body<NT, F_WEIERSTRASS, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_SCHWEFEL: wide_body<NT, F_SCHWEFEL, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_ELLIPTIC: wide_body<NT, F_ELLIPTIC, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_REF_ACKLEY: wide_body<NT, F_REF_ACKLEY, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_REF_RASTRIGIN: wide_body<NT, F_REF_RASTRIGIN, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_REF_GRIEWANK: case F_REF_GRIEWANK_GA: wide_body<NT, F_REF_GRIEWANK, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_REF_WEIERSTRASS: wide_body<NT, F_REF_WEIERSTRASS, ALGO, WT, QL>(a, smem, task, td); break;
-    case F_REF_SCHWEFEL: wide_body<NT, F_SCHWEFEL, ALGO, WT, QL>(a, smem, task, td); break;
+    case F_SPHERE: wide_body<NT, F_SPHERE, ALGO, QL>(a, smem, task, td); break;
+    case F_ROSENBROCK: wide_body<NT, F_ROSENBROCK, ALGO, QL>(a, smem, task, td); break;
+    case F_ACKLEY: wide_body<NT, F_ACKLEY, ALGO, QL>(a, smem, task, td); break;
+    case F_RASTRIGIN: wide_body<NT, F_RASTRIGIN, ALGO, QL>(a, smem, task, td); break;
+    case F_GRIEWANK: wide_body<NT, F_GRIEWANK, ALGO, QL>(a, smem, task, td); break;
+    case F_WEIERSTRASS: wide_body<NT, F_WEIERSTRASS, ALGO, QL>(a, smem, task, td); break;
+    case F_SCHWEFEL: wide_body<NT, F_SCHWEFEL, ALGO, QL>(a, smem, task, td); break;
+    case F_ELLIPTIC: wide_body<NT, F_ELLIPTIC, ALGO, QL>(a, smem, task, td); break;
+    case F_REF_ACKLEY: wide_body<NT, F_REF_ACKLEY, ALGO, QL>(a, smem, task, td); break;
+    case F_REF_RASTRIGIN: wide_body<NT, F_REF_RASTRIGIN, ALGO, QL>(a, smem, task, td); break;
+    case F_REF_GRIEWANK: case F_REF_GRIEWANK_GA: wide_body<NT, F_REF_GRIEWANK, ALGO, QL>(a, smem, task, td); break;
+    case F_REF_WEIERSTRASS: wide_body<NT, F_REF_WEIERSTRASS, ALGO, QL>(a, smem, task, td); break;
+    case F_REF_SCHWEFEL: wide_body<NT, F_SCHWEFEL, ALGO, QL>(a, smem, task, td); break;
     default: break;
     }
 }
-
 #endif  // EMTF_WIDE_NT
 
 }  // namespace emtf
@@ -1883,49 +2048,43 @@ __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
 #define EMTF_WCAT(a, b, c, d) a##b##_##c##d
 #define EMTF_WNAME(a, b, c, d) EMTF_WCAT(a, b, c, d)
 
-// Wide-task LDS: o, table, fitness, scratch fitness, ranks, flags.
+// The Q image in LDS where it fits beside the population's arrays: every population up to
+// 1024 for NT <= 5, up to 512 for NT = 6; else read from L2.
+static bool wide_q_in_lds(int pop) {
+    return EMTF_WIDE_NT <= 6 && 4 * emtf::wide_lds_floats(EMTF_WIDE_NT, pop, true) <= 160 * 1024;
+}
+
 extern "C" int EMTF_WNAME(emtf_wide_lds_floats_nt, EMTF_WIDE_NT, a, EMTF_ALGO)(int pop) {
-    const int popP = (pop + 31) & ~31;
-    return emtf::WShape<EMTF_WIDE_NT>::RS + 32 * EMTF_WIDE_NT + 4 * popP;
+    return emtf::wide_lds_floats(EMTF_WIDE_NT, pop, wide_q_in_lds(pop));
 }
 
-extern "C" int EMTF_WNAME(emtf_launch_wide_nt, EMTF_WIDE_NT, a, EMTF_ALGO)(const emtf::EpochArgs* args, const int* order,
-                                                                          int n, int lds_bytes, hipStream_t stream) {
-    hipLaunchKernelGGL((emtf::wide_epoch_kernel<EMTF_WIDE_NT, EMTF_ALGO, 256, false, emtf::kWideWpe>), dim3(n), dim3(256), lds_bytes, stream,
-                       *args, order);
-    return (int)hipGetLastError();
-}
-
-extern "C" int EMTF_WNAME(emtf_launch_wide8_nt, EMTF_WIDE_NT, a, EMTF_ALGO)(const emtf::EpochArgs* args, const int* order,
-                                                                           int n, int lds_bytes, hipStream_t stream) {
-    hipLaunchKernelGGL((emtf::wide_epoch_kernel<EMTF_WIDE_NT, EMTF_ALGO, 512, false, emtf::kWideWpe>), dim3(n), dim3(512), lds_bytes, stream,
-                       *args, order);
-    return (int)hipGetLastError();
-}
-
-// 512 threads with the Q image in LDS (lds_bytes includes it): built where it fits
-#if EMTF_WIDE_NT <= 6
-extern "C" int EMTF_WNAME(emtf_launch_wideq_nt, EMTF_WIDE_NT, a, EMTF_ALGO)(const emtf::EpochArgs* args, const int* order,
-                                                                           int n, int lds_bytes, hipStream_t stream) {
+template <bool QL>
+static hipError_t launch_wide(const emtf::EpochArgs& a, const int* order, int n, int lds_bytes, hipStream_t stream) {
     static bool lds_ok = false;
-    auto k = &emtf::wide_epoch_kernel<EMTF_WIDE_NT, EMTF_ALGO, 512, true, emtf::kWideWpe>;
+    auto k = &emtf::wide_epoch_kernel<EMTF_WIDE_NT, EMTF_ALGO, QL>;
     if (!lds_ok) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        if (e != hipSuccess) return (int)e;
+        if (e != hipSuccess) return e;
         lds_ok = true;
     }
-    hipLaunchKernelGGL(k, dim3(n), dim3(512), lds_bytes, stream, *args, order);
-    return (int)hipGetLastError();
+    hipLaunchKernelGGL(k, dim3(n), dim3(emtf::kWideThreads), lds_bytes, stream, a, order);
+    return hipGetLastError();
 }
 
-extern "C" int EMTF_WNAME(emtf_wideq_lds_floats_nt, EMTF_WIDE_NT, a, EMTF_ALGO)(int pop) {
-    const int popP = (pop + 31) & ~31;
-    using S = emtf::WShape<EMTF_WIDE_NT>;
-    return 32 * EMTF_WIDE_NT * S::RS + S::RS + 32 * EMTF_WIDE_NT + 4 * popP;
-}
+// lds_bytes: 4 emtf_wide_lds_floats of the unit's largest population, which says whether the Q
+// image is in it.
+extern "C" int EMTF_WNAME(emtf_launch_wide_nt, EMTF_WIDE_NT, a, EMTF_ALGO)(const emtf::EpochArgs* args, const int* order,
+                                                                          int n, int lds_bytes, hipStream_t stream) {
+#if EMTF_WIDE_NT <= 6
+    if (lds_bytes >= 4 * 1024 * EMTF_WIDE_NT * EMTF_WIDE_NT) return (int)launch_wide<true>(*args, order, n, lds_bytes, stream);
 #endif
-
+#if EMTF_WIDE_NT >= 6
+    return (int)launch_wide<false>(*args, order, n, lds_bytes, stream);
+#else
+    return (int)hipErrorInvalidValue;
+#endif
+}
 #else
 #if !defined(EMTF_KB) || !defined(EMTF_ALGO)
 #error "compile island.hip with -DEMTF_KB=<gene blocks per half> -DEMTF_ALGO=<0|2>"

@@ -473,3 +473,29 @@ def test_ga_boxes_and_exponents(oracle_mod, box, eta_c, eta_m, pm):
     gpu.run(6)
     orc.run(6)
     _compare(gpu, orc, f"GA box {box} eta {eta_c}, {eta_m}")
+
+
+@pytest.mark.parametrize("pop", [2, 32, 33, 64, 96, 128, 129, 256, 288])
+def test_wide_row_tiles_split_over_waves(oracle_mod, pop):
+    """Populations on both sides of each split of a tile's row tiles over 8, 4, 2 and 1 waves,
+    at every row tile count, every objective, generations in odd and even runs."""
+    dims = [100, 129, 160, 161, 192, 193, 224, 225, 256]
+    funcs = [tg.FUNC_IDS[f] for f in tg.CYCLE]
+    tasks = []
+    for k, d in enumerate(dims):
+        tasks += tg.benchmark_tasks(3, d, pop, rotate=True, seed=55 + k, funcs=[funcs[(3 * k + j) % 8] for j in range(3)])
+    gpu, orc = _pair(tasks, oracle_mod, seed=5, tune=2, transfer_interval=4, transfer_count=1)
+    for step in (1, 3, 2):
+        gpu.run(step)
+        orc.run(step)
+        _compare(gpu, orc, f"wide pop {pop} gen {orc.generation}")
+
+
+@pytest.mark.parametrize("pop", [512, 544])
+def test_wide_q_beside_the_largest_population(oracle_mod, pop):
+    """D = 192: the largest population whose arrays fit LDS beside the task's Q, and the next."""
+    tasks = tg.benchmark_tasks(2, 192, pop, rotate=True, seed=57)
+    gpu, orc = _pair(tasks, oracle_mod, seed=7)
+    gpu.run(2)
+    orc.run(2)
+    _compare(gpu, orc, f"NT 6 pop {pop}")

@@ -143,3 +143,26 @@ def test_gpu_reference_formulas_bit_exact(oracle_mod, formulas, algo, D):
             xo, fo = orc.population(t)
             assert np.array_equal(fg.view(np.uint32), fo.view(np.uint32)), (step, t, tasks[t]["func"])
             assert np.array_equal(xg.view(np.uint32), xo.view(np.uint32)), (step, t)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("formulas, algo", [(1, 1), (2, 2)])
+@pytest.mark.parametrize("pop", [32, 64, 128, 160])
+def test_gpu_reference_formulas_over_split_row_tiles(oracle_mod, formulas, algo, pop):
+    """The reference's formulas with a tile's row tiles on 8, 4, 2 and 1 waves (their sums
+    carried from wave to wave)."""
+    import emtf
+    tasks = _ref_tasks(14, 170, pop, seed=pop)
+    ga = formulas == 2
+    params = dict(seed=11, algo=algo, F=0.5, CR=0.6, n_islands=4, exchange_interval=2, migrate_interval=3,
+                  migrate_count=2, transfer_interval=4, transfer_count=2, transfer_cr=0.4)
+    print(f"case: reference formulas {formulas} algo {algo} pop {pop}", flush=True)
+    gpu = emtf.Engine(tasks, formulas=formulas, **params)
+    orc = oracle_mod.Engine([dict(t, func=ref_id(t["func"], ga)) for t in tasks], **params)
+    gpu.run(9)
+    orc.run(9)
+    for t in range(len(tasks)):
+        xg, fg = gpu.population(t)
+        xo, fo = orc.population(t)
+        assert np.array_equal(fg.view(np.uint32), fo.view(np.uint32)), (t, tasks[t]["func"])
+        assert np.array_equal(xg.view(np.uint32), xo.view(np.uint32)), t
