@@ -34,7 +34,8 @@
 #define EMTF_DECL_PAIR(kb) EMTF_DECL_LAUNCH(kb, 0) EMTF_DECL_LAUNCH(kb, 2)
 EMTF_DECL_PAIR(2) EMTF_DECL_PAIR(4) EMTF_DECL_PAIR(7) EMTF_DECL_PAIR(8) EMTF_DECL_PAIR(12) EMTF_DECL_PAIR(13)
 EMTF_DECL_PAIR(16)
-extern "C" int emtf_lds_floats_kb(int pop, int kb);
+extern "C" int emtf_lds_floats_kb(int pop, int kb);        // population and Q: the rule for the LDS kernel
+extern "C" int emtf_epoch_lds_floats_kb(int pop, int kb);  // what its launch allocates
 #define EMTF_DECL_WIDE(nt, al)                                                                             \
     extern "C" int emtf_launch_wide_nt##nt##_a##al(const emtf::EpochArgs* args, const int* order, int n,   \
                                                    int lds_bytes, hipStream_t stream);                     \
@@ -212,7 +213,7 @@ struct emtf_handle {
     float* d_tab = nullptr;
     float* d_mailbox = nullptr;
     float* d_scratch = nullptr;
-    float* d_qw = nullptr;       // Q images in operand order of the wide kernel
+    float* d_qw = nullptr;       // Q images in operand order (wide kernel; LDS kernel from KB = 12)
     int* d_order = nullptr;      // task ids grouped by bucket
     std::vector<Bucket> buckets;
     bool polish = false;
@@ -755,7 +756,7 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
     // bucket of every task: LDS kernel of the smallest KB whose population fits, else the wide kernel
     const bool ga = prm->algo == EMTF_GA_SBX_PM;
     const bool want_polish = prm->polish_interval > 0 && prm->polish_steps > 0 && prm->polish_topk > 0;
-    std::vector<int> bucket_of(n_tasks), wide_nt(n_tasks, -1);
+    std::vector<int> bucket_of(n_tasks), wide_nt(n_tasks, -1), image_nt(n_tasks, 0);
     std::vector<double> cost(n_tasks);
     for (int t = 0; t < n_tasks; ++t) {
         const emtf_task_desc& d = tasks[t];
@@ -797,7 +798,7 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
             pick_wide(geo, ga, &wl);
             b.lds_bytes = std::max(b.lds_bytes, 4 * wl(d.pop));
         } else {
-            b.lds_bytes = std::max(b.lds_bytes, 4 * emtf_lds_floats_kb(d.pop, geo));
+            b.lds_bytes = std::max(b.lds_bytes, 4 * emtf_epoch_lds_floats_kb(d.pop, geo));
         }
         // relative cost per generation: objective work per gene + the rotation GEMM
         const int dk = wide ? 32 * geo : 8 * geo;
@@ -885,8 +886,10 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
         if (wide_nt[t] > 0) {
             const int RS = 32 * wide_nt[t] + 4;
             scr = std::max(scr, 2 * (int64_t)popP * RS);  // population rows, trial rows
-            nW += (int64_t)1024 * wide_nt[t] * wide_nt[t];
         }
+        // the wide kernel's row tiles; four for the LDS kernel (a wide variant's are the same there)
+        image_nt[t] = wide_nt[t] > 0 ? wide_nt[t] : (!b.wide && b.geo >= 12 ? 4 : 0);
+        nW += (int64_t)1024 * image_nt[t] * image_nt[t];
         nS += scr;
     }
     for (size_t k = 0; k < h->buckets.size(); ++k)
@@ -1067,7 +1070,7 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
     int* d_nt = nullptr;  // row tiles of the tasks with a Q image; freed after the synchronisation below
     if (nW > 0) {
         e = hipMalloc((void**)&d_nt, sizeof(int) * n_tasks);
-        if (e == hipSuccess) e = hipMemcpy(d_nt, wide_nt.data(), sizeof(int) * n_tasks, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(d_nt, image_nt.data(), sizeof(int) * n_tasks, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = (hipError_t)emtf_launch_q_images(h->d_tasks, d_nt, n_tasks, h->d_Q, h->d_qw, nullptr);
         if (e != hipSuccess) { (void)hipFree(d_nt); free_handle(h); return fail(EMTF_E_DEVICE, std::string("Q images: ") + hipGetErrorString(e)); }
     }

@@ -61,6 +61,15 @@ __device__ __forceinline__ float4 q_op(const float* q, int nt, int sb, int jt) {
     return make_float4(p[0], p[1], p[2], p[3]);
 }
 
+// LDS-kernel builds that read Q's image (of kQTiles row tiles) from L2, a block ahead of its
+// use: from KB = 12 on the rows and Q together leave room for one workgroup a CU, a wave per
+// SIMD that issues an instruction each 5.7 cycles; the rows alone for two.  D = 100, pop 128, an
+// epoch of 20 generations: 1024 sphere tasks 1.145 to 0.826 ms, Weierstrass 3.66 to 1.77; 256
+// tasks (one workgroup a CU either way) 0.312 to 0.281 and 0.945 to 0.719.
+template <int KB>
+constexpr bool kQGlobal = KB >= 12;
+constexpr int kQTiles = 4;
+
 struct Geo {
     int D, Dh, pop, popP, ntiles, m;
     FastMod modD, modM;  // jrand = w mod D, island-local index = w mod m
@@ -80,6 +89,11 @@ struct Lds {
 __host__ __device__ inline int lds_floats_kb(int pop, int kb) {
     const int RS = 8 * kb + 4, NT = (kb + 3) / 4, popP = (pop + 31) & ~31;
     return popP * RS + 32 * NT * RS + RS + 32 * NT + 4 * popP;
+}
+
+// What the epoch kernel allocates: the same, without Q where it reads the image.
+__host__ __device__ inline int epoch_lds_floats(int pop, int kb) {
+    return lds_floats_kb(pop, kb) - (kb >= 12 ? 32 * ((kb + 3) / 4) * (8 * kb + 4) : 0);
 }
 
 // v clamped to [lo, hi] (hi if v > hi, else lo if v < lo, else v: a NaN stays NaN), as
@@ -156,13 +170,14 @@ __device__ __forceinline__ float evaluate_tile(const float (&x)[4 * KB], const G
     for (int jt = 0; jt < NT; ++jt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[jt][r] = 0.0f;
-    const float* qrow = L.Q + col * S::RS + h * S::HS;
+    const float* qrow = kQGlobal<KB> ? L.Q + 4 * (32 * h + col) : L.Q + col * S::RS + h * S::HS;
     const float* orow = L.o + h * S::HS;
 #pragma unroll
     for (int sb = 0; sb < KB; ++sb) {
         float4 q[NT];
 #pragma unroll
-        for (int jt = 0; jt < NT; ++jt) q[jt] = lds4(qrow + 32 * jt * S::RS + 4 * sb);
+        for (int jt = 0; jt < NT; ++jt)
+            q[jt] = kQGlobal<KB> ? q_op(qrow, kQTiles, sb, jt) : lds4(qrow + 32 * jt * S::RS + 4 * sb);
         const float4 o4 = lds4(orow + 4 * sb);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -541,8 +556,13 @@ __device__ __forceinline__ float trial_eval(float (&tr)[4 * KB], const EpochArgs
     for (int jt = 0; jt < NT; ++jt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[jt][r] = 0.0f;
-    const float* qrow = L.Q + col * S::RS + off;
+    const float* qrow = kQGlobal<KB> ? L.Q + 4 * (32 * h + col) : L.Q + col * S::RS + off;
     const float* orow = L.o + off;
+    float4 qn[NT];  // the next block's, loaded a block ahead from L2
+    if constexpr (kQGlobal<KB>) {
+#pragma unroll
+        for (int jt = 0; jt < NT; ++jt) qn[jt] = q_op(qrow, kQTiles, 0, jt);
+    }
     // GA: the pair's mates and constants; DE: the three mates and jrand
     const float *p0, *p1, *p2, *p3;
     bool odd = false;
@@ -592,7 +612,14 @@ __device__ __forceinline__ float trial_eval(float (&tr)[4 * KB], const EpochArgs
         }
         float4 q[NT];
 #pragma unroll
-        for (int jt = 0; jt < NT; ++jt) q[jt] = lds4(qrow + 32 * jt * S::RS + 4 * sb);
+        for (int jt = 0; jt < NT; ++jt) {
+            if constexpr (kQGlobal<KB>) {
+                q[jt] = qn[jt];
+                if (sb + 1 < KB) qn[jt] = q_op(qrow, kQTiles, sb + 1, jt);
+            } else {
+                q[jt] = lds4(qrow + 32 * jt * S::RS + 4 * sb);
+            }
+        }
         const float4 o4 = lds4(orow + 4 * sb);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -611,7 +638,7 @@ __device__ __forceinline__ float trial_eval(float (&tr)[4 * KB], const EpochArgs
     }
     // the padded row groups are skipped for the two costliest epilogues only (measured:
     // the branch costs more than it saves for the others)
-    // Q's rows past D are zero in LDS (zeroed at the epoch's start)
+    // Q's rows past D are zero (in LDS zeroed at the epoch's start)
     return objective<NT, FUNC, FUNC == F_WEIERSTRASS || FUNC == F_SCHWEFEL || FUNC == F_REF_WEIERSTRASS, true>(
         acc, g.D, L.tab, h);
 }
@@ -1274,8 +1301,8 @@ __device__ __forceinline__ void epoch_body(const EpochArgs& a, float* smem, cons
     g.modM.init((uint32_t)g.m);
     Lds L;
     L.X = smem;
-    L.Q = L.X + g.popP * RS;
-    L.o = L.Q + 32 * NT * RS;
+    L.Q = kQGlobal<KB> ? const_cast<float*>(a.Qw + td.qw_off) : L.X + g.popP * RS;
+    L.o = kQGlobal<KB> ? L.X + g.popP * RS : L.Q + 32 * NT * RS;
     L.tab = L.o + RS;
     L.fit = L.tab + 32 * NT;
     L.ftmp = L.fit + g.popP;
@@ -1287,7 +1314,7 @@ __device__ __forceinline__ void epoch_body(const EpochArgs& a, float* smem, cons
     const int nz = L.fit - smem;  // X, Q, o, tab
     for (int e = tid; e < nz; e += kThreads) smem[e] = 0.0f;
     __syncthreads();
-    stage_rows<RS, HS>(L.Q, a.Q + td.q_off, g.D, g.D, tid);
+    if constexpr (!kQGlobal<KB>) stage_rows<RS, HS>(L.Q, a.Q + td.q_off, g.D, g.D, tid);
     for (int d = tid; d < g.D; d += kThreads) {
         L.o[(d & 1) * HS + (d >> 1)] = a.shift[td.v_off + d];
         L.tab[d] = a.tab[td.v_off + d];
@@ -1360,10 +1387,14 @@ __device__ __forceinline__ void epoch_body(const EpochArgs& a, float* smem, cons
 // One workgroup per task; `order` lists the tasks longest-first so the
 // expensive objectives are dispatched before the cheap ones fill the gaps.
 // Register budget: with KB <= 8 (dims <= 64) three 4-wave workgroups fit in LDS per
-// CU, so the allocator is asked for 3 waves per SIMD (<= 168 VGPR+AGPR); larger
-// rows are LDS-bound to fewer workgroups and keep the default budget.
-#if !defined(EMTF_WAVES_PER_EU) && defined(EMTF_KB) && EMTF_KB <= 8
+// CU, so the allocator is asked for 3 waves per SIMD (<= 168 VGPR+AGPR); of the larger
+// rows two fit (256).
+#if !defined(EMTF_WAVES_PER_EU) && defined(EMTF_KB)
+#if EMTF_KB <= 8
 #define EMTF_WAVES_PER_EU 3
+#else
+#define EMTF_WAVES_PER_EU 2
+#endif
 #endif
 #ifdef EMTF_WAVES_PER_EU
 #define EMTF_OCCUPANCY __attribute__((amdgpu_waves_per_eu(EMTF_WAVES_PER_EU, EMTF_WAVES_PER_EU)))
@@ -2136,6 +2167,7 @@ extern "C" int EMTF_NAME(emtf_launch_persist_kb, EMTF_KB, a, EMTF_ALGO)(const em
 
 #if EMTF_KB == 2 && EMTF_ALGO == 0
 extern "C" int emtf_lds_floats_kb(int pop, int kb) { return emtf::lds_floats_kb(pop, kb); }
+extern "C" int emtf_epoch_lds_floats_kb(int pop, int kb) { return emtf::epoch_lds_floats(pop, kb); }
 #endif
 
 #if EMTF_ALGO == 0
