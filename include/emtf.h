@@ -92,8 +92,10 @@ enum { EMTF_FORMULAS_TEXTBOOK = 0, EMTF_FORMULAS_REFERENCE_DE = 1, EMTF_FORMULAS
 /* How emtf_run launches work.  Work is cut into epochs that end at every transfer
  * boundary, the kernel boundary ordering the elite mailbox.  EPOCHS: each epoch's kernels
  * (one per launch unit, forked over up to four streams and joined) are launched directly.
- * AUTO: the same epochs, replayed from a hipGraph that the handle captures once (and again
- * when the epoch length changes): epochs of one whole transfer interval (or of any length
+ * AUTO: the same epochs; with several launch units (or while the caller captures the stream)
+ * they are replayed from a hipGraph that the handle captures once (and again when the epoch
+ * length changes), with one launch unit its one kernel is launched directly.  Replayed are
+ * epochs of one whole transfer interval (or of any length
  * without transfer) whose end carries no trace point or polish; the kernels read their
  * first generation from a device counter that the graph advances.  Same results either way.
  * PERSISTENT: one launch per call (per stretch between trace points, at most 1024 epochs

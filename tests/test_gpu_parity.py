@@ -499,3 +499,19 @@ def test_wide_q_beside_the_largest_population(oracle_mod, pop):
     gpu.run(2)
     orc.run(2)
     _compare(gpu, orc, f"NT 6 pop {pop}")
+
+
+@pytest.mark.parametrize("n_tasks", [240, 250])
+def test_elites_on_both_sides_of_the_pinned_size(n_tasks):
+    """Elite exports of 16 (1 + 67) floats a task, just within and beyond 2^18 floats: equal to
+    the populations' best rows."""
+    tasks = tg.benchmark_tasks(n_tasks, 67, 16, rotate=False, seed=58)
+    gpu = emtf.Engine(tasks, seed=8)
+    gpu.run(3)
+    for k in (1, 16):
+        f, x = gpu.elites(k)
+        for t in (0, n_tasks // 2, n_tasks - 1):
+            xp, fp = gpu.population(t)
+            order = np.argsort(fp, kind="stable")[:k]
+            assert np.array_equal(f[t], fp[order]), f"task {t} k {k}"
+            assert np.array_equal(x[t][:, :67], xp[order]), f"task {t} k {k}"
