@@ -1475,8 +1475,8 @@ __global__ __launch_bounds__(kThreads) EMTF_OCCUPANCY void island_persistent_ker
         }
         __syncthreads();
         if (!s_ok) return;  // the error flag is set: the launch drains
-        // (the waits' acquire loads and the stamp's release store, with the workgroup
-        // barriers around them, order the rows, fitness and mailbox across workgroups)
+        // (the waits' acquire loads and the stamp's release store, with the fence and the
+        // workgroup barriers around them, order the rows, fitness and mailbox across workgroups)
         switch (td.func) {
         case F_SPHERE: epoch_body<KB, F_SPHERE, ALGO, true>(a, smem, task, td, &pa, e, g0, g1, pub); break;
         case F_ROSENBROCK: epoch_body<KB, F_ROSENBROCK, ALGO, true>(a, smem, task, td, &pa, e, g0, g1, pub); break;
@@ -1495,6 +1495,9 @@ __global__ __launch_bounds__(kThreads) EMTF_OCCUPANCY void island_persistent_ker
         case F_REF_SCHWEFEL: epoch_body<KB, F_SCHWEFEL, ALGO, true>(a, smem, task, td, &pa, e, g0, g1, pub); break;
         default: break;
         }
+        // every wave's rows, fitness and elites are in memory before the stamp: the barrier
+        // alone does not wait for the other waves' stores
+        __threadfence();
         __syncthreads();
         if (tid == 0 && __hip_atomic_load(pa.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
             __hip_atomic_store(pa.stamp + task, e + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
