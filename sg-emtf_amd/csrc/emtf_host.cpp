@@ -1038,8 +1038,10 @@ int emtf_create(const emtf_task_desc* tasks, int32_t n_tasks, const emtf_params*
         return EMTF_OK;
     };
     int rc = EMTF_OK;
-    if ((rc = alloc(&h->d_X, nX)) || (rc = alloc(&h->d_fit, nF)) || (rc = alloc(&h->d_Q, nQ)) ||
-        (rc = alloc(&h->d_shift, nV)) || (rc = alloc(&h->d_tab, nV)) || (rc = alloc(&h->d_mailbox, 2 * h->mailbox_stride)) ||
+    // X and Q: eight floats longer, for the kernels' wide loads of a row's last block; the
+    // mailbox: 128, for loads of as many genes as a kernel build holds
+    if ((rc = alloc(&h->d_X, nX + 8)) || (rc = alloc(&h->d_fit, nF)) || (rc = alloc(&h->d_Q, nQ + 8)) ||
+        (rc = alloc(&h->d_shift, nV)) || (rc = alloc(&h->d_tab, nV)) || (rc = alloc(&h->d_mailbox, 2 * h->mailbox_stride + 128)) ||
         (rc = alloc(&h->d_scratch, nS)) || (rc = alloc(&h->d_qw, nW))) {
         free_handle(h);
         return rc;

@@ -643,25 +643,94 @@ __device__ __forceinline__ float trial_eval(float (&tr)[4 * KB], const EpochArgs
         acc, g.D, L.tab, h);
 }
 
-// Copies an n x D row-major matrix from global memory into LDS rows of stride RS in the
-// [even | odd] gene layout (gene d at (d & 1) HS + d / 2), eight loads in flight per
-// thread, so a load's latency is paid once per eight elements rather than per element.
-template <int RS, int HS>
-__device__ __forceinline__ void stage_rows(float* dst, const float* __restrict__ src, int n, int D, int tid) {
-    const int total = n * D;
-    for (int e0 = tid; e0 < total; e0 += 8 * kThreads) {
-        float v[8];
+// Sixteen bytes at any float's address.
+struct __attribute__((packed, aligned(4))) F4U {
+    float x, y, z, w;
+};
+
+// Rows of an n x D row-major matrix in global memory to np rows of stride RS in the [even | odd]
+// layout (gene d at (d & 1) HS + d / 2), nb blocks of eight genes each; zeros past the
+// dimension and past row n.  A thread takes a block: two 16-byte loads and two 16-byte stores, B
+// blocks in flight, so an epoch's start costs a latency or two and no division per gene.  A
+// row's last block reads up to seven floats past the row: the arrays are allocated eight longer.
+// What an epoch costs beside its generations (256 tasks, pop 128; with the ranking and the
+// transfer): D = 50 29 to 24 us, D = 150 (wide kernel) 63 to 47.
+template <int RS, int HS, int NTHR, int B>
+__device__ __forceinline__ void stage_rows(float* dst, const float* __restrict__ src, int n, int np, int D, int nb,
+                                           int tid) {
+    const int di = NTHR / nb, dk = NTHR - di * nb;
+    int i = tid / nb, k = tid - i * nb;
+    while (i < np) {
+        F4U v[B][2];
+        int ii[B], kk[B];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int e = e0 + k * kThreads;
-            v[k] = e < total ? src[e] : 0.0f;
+        for (int b = 0; b < B; ++b) {
+            ii[b] = i;
+            kk[b] = k;
+            const F4U* s = reinterpret_cast<const F4U*>(src + (i < n && 8 * k < D ? (int64_t)i * D + 8 * k : 0));
+            v[b][0] = s[0];
+            v[b][1] = s[1];
+            i += di;
+            k += dk;
+            if (k >= nb) {
+                k -= nb;
+                ++i;
+            }
         }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int e = e0 + k * kThreads;
-            if (e < total) {
-                const int j = e / D, d = e - j * D;
-                dst[j * RS + (d & 1) * HS + (d >> 1)] = v[k];
+        for (int b = 0; b < B; ++b) {
+            if (ii[b] >= np) break;
+            const int left = ii[b] < n ? D - 8 * kk[b] : 0;  // genes of the block
+            const float4 ev = make_float4(left > 0 ? v[b][0].x : 0.0f, left > 2 ? v[b][0].z : 0.0f,
+                                          left > 4 ? v[b][1].x : 0.0f, left > 6 ? v[b][1].z : 0.0f);
+            const float4 od = make_float4(left > 1 ? v[b][0].y : 0.0f, left > 3 ? v[b][0].w : 0.0f,
+                                          left > 5 ? v[b][1].y : 0.0f, left > 7 ? v[b][1].w : 0.0f);
+            float* row = dst + (int64_t)ii[b] * RS + 4 * kk[b];
+            *reinterpret_cast<float4*>(row) = ev;
+            *reinterpret_cast<float4*>(row + HS) = od;
+        }
+    }
+}
+
+// The way back: n rows, row i at src + row(i), to an n x D row-major matrix.
+template <int HS, int NTHR, int B, typename Row>
+__device__ __forceinline__ void unstage_rows(float* __restrict__ dst, const float* src, Row row, int n, int D, int tid) {
+    const int nb = (D + 7) >> 3, di = NTHR / nb, dk = NTHR - di * nb;
+    int i = tid / nb, k = tid - i * nb;
+    while (i < n) {
+        float4 ev[B], od[B];
+        int ii[B], kk[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            ii[b] = i;
+            kk[b] = k;
+            const float* r = src + (i < n ? row(i) + 4 * k : row(0));
+            ev[b] = lds4(r);
+            od[b] = lds4(r + HS);
+            i += di;
+            k += dk;
+            if (k >= nb) {
+                k -= nb;
+                ++i;
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            if (ii[b] >= n) break;
+            const int left = D - 8 * kk[b];
+            float* o = dst + (int64_t)ii[b] * D + 8 * kk[b];
+            const F4U lo{ev[b].x, od[b].x, ev[b].y, od[b].y}, hi{ev[b].z, od[b].z, ev[b].w, od[b].w};
+            if (left >= 8) {
+                reinterpret_cast<F4U*>(o)[0] = lo;
+                reinterpret_cast<F4U*>(o)[1] = hi;
+            } else {
+                o[0] = lo.x;
+                if (left > 1) o[1] = lo.y;
+                if (left > 2) o[2] = lo.z;
+                if (left > 3) o[3] = lo.w;
+                if (left > 4) o[4] = hi.x;
+                if (left > 5) o[5] = hi.y;
+                if (left > 6) o[6] = hi.z;
             }
         }
     }
@@ -688,18 +757,24 @@ __device__ __forceinline__ void store_half_row(float* row, const float (&x)[4 * 
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float key_of(float f) { return (f != f) ? __builtin_inff() : f; }
 
-// ord[q m + rank] = i: the members of each island q ranked by (fitness, index)
+// ord[q m + rank] = i: the members of each island q ranked by (fitness, index).  Threads to
+// spare share an individual's comparisons, two to eight adjacent lanes each.
 template <int NTHR = kThreads>
 __device__ __forceinline__ void rank_islands(const Lds& L, int pop, int m, int tid) {
-    for (int i = tid; i < pop; i += NTHR) {
+    int sh = 0;
+    while (sh < 3 && (pop << (sh + 1)) <= NTHR) ++sh;
+    for (int t = tid; t < (pop << sh); t += NTHR) {
+        const int i = t >> sh;
         const int q = i / m, base = q * m, il = i - base;
         const float fi = key_of(L.fit[i]);
         int r = 0;
-        for (int p = 0; p < m; ++p) {
+#pragma unroll 8
+        for (int p = t & ((1 << sh) - 1); p < m; p += 1 << sh) {
             const float fp = key_of(L.fit[base + p]);
             r += (fp < fi || (fp == fi && p < il)) ? 1 : 0;
         }
-        L.ord[base + r] = i;
+        for (int d = 1; d < (1 << sh); d <<= 1) r += __shfl_xor(r, d);
+        if ((t & ((1 << sh) - 1)) == 0) L.ord[base + r] = i;
     }
 }
 
@@ -842,27 +917,45 @@ __device__ __forceinline__ void transfer_in(const EpochArgs& a, const TaskDev& t
         const int j = ct * 32 + col;
         const bool valid = j < k;
         const int je = valid ? j : 0;
+        // the donor's genes (of the build's every slot: the mailbox is allocated a longest row
+        // longer), then the box and the draws where they matter, then one select a gene:
+        // straight code, since every epoch fetches it anew
+        const float* mrow = mb + (int64_t)je * dd.dim;
+        const int dlim = (g.D < dd.dim ? g.D : dd.dim) - h;  // gene 2 q + h is transferable
+        const float* own = L.X + L.ord[je] * S::RS + h * S::HS;
         float cand[S::HS];
-        load_half_row<KB>(cand, L.X + L.ord[je] * S::RS + h * S::HS);
+        constexpr int VB = S::HS < 32 ? S::HS : 32;
 #pragma unroll
-        for (int s = 0; s < S::HS; ++s) {
-            const int d = 2 * s + h;
-            if (d < g.D && d < dd.dim) {
-                bool take = true;
-                if (a.p.transfer_cr > 0.0f) {
-                    const uint32_t wu = rng.word((uint32_t)g0, P_XFER, (uint32_t)je, (uint32_t)h, (uint32_t)s);
-                    take = uniform01(wu) > a.p.transfer_cr;
+        for (int q0 = 0; q0 < S::HS; q0 += VB) {
+            float v[VB];
+#pragma unroll
+            for (int r = 0; r < VB; ++r) v[r] = mrow[2 * (q0 + r) + h];
+            if (!same_box) {
+#pragma unroll
+                for (int r = 0; r < VB; ++r) {
+                    const float t1 = v[r] - dd.lo;
+                    const float t2 = t1 / rng_d;
+                    const float t3 = t2 * rng_s;
+                    v[r] = td.lo + t3;
                 }
-                if (take) {
-                    const float v = mb[(int64_t)je * dd.dim + d];
-                    if (same_box) cand[s] = v;
-                    else {
-                        const float t1 = v - dd.lo;
-                        const float t2 = t1 / rng_d;
-                        const float t3 = t2 * rng_s;
-                        cand[s] = td.lo + t3;
-                    }
+            }
+            uint32_t take = 0xFFFFFFFFu;
+            if (a.p.transfer_cr > 0.0f) {
+                take = 0u;
+#pragma unroll 1
+                for (int b = 0; b < VB / 4; ++b) {
+                    const U4 ub = rng.block((uint32_t)g0, P_XFER, (uint32_t)je, (uint32_t)h, (uint32_t)(q0 / 4 + b));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        take |= uniform01(pick(ub, (uint32_t)e)) > a.p.transfer_cr ? 1u << (4 * b + e) : 0u;
                 }
+            }
+#pragma unroll
+            for (int r = 0; r < VB && q0 + r < S::HS; r += 4) {
+                const float4 o4 = lds4(own + q0 + r);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    cand[q0 + r + e] = (2 * (q0 + r + e) < dlim && ((take >> (r + e)) & 1u)) ? v[r + e] : f4(o4, e);
             }
         }
         const float f = evaluate_tile<KB, FUNC>(cand, g, L, col, h);
@@ -951,13 +1044,10 @@ __device__ __forceinline__ void polish_body(const EpochArgs& a, float* smem, con
     float* const PS = slots + nsl * PSZ;  // the line search's running row sums, s1 | s2 per lane
     float* const PZ = PS + 128;           // Rosenbrock: row 0 of each tile per candidate
     static_assert(NT <= NW, "one row tile per wave in the line search");
-    const int nz = 32 * NT * RS + RS + 32 * NT;
-    for (int e = tid; e < nz; e += kThreads) smem[e] = 0.0f;
-    __syncthreads();
-    stage_rows<RS, HS>(L.Q, a.Q + td.q_off, g.D, g.D, tid);
-    for (int d = tid; d < g.D; d += kThreads) {
-        L.o[(d & 1) * HS + (d >> 1)] = a.shift[td.v_off + d];
-        L.tab[d] = a.tab[td.v_off + d];
+    stage_rows<RS, HS, kThreads, 4>(L.Q, a.Q + td.q_off, g.D, 32 * NT, g.D, KB, tid);
+    for (int d = tid; d < 32 * NT; d += kThreads) {
+        if (d < 2 * HS) L.o[(d & 1) * HS + (d >> 1)] = d < g.D ? a.shift[td.v_off + d] : 0.0f;
+        L.tab[d] = d < g.D ? a.tab[td.v_off + d] : 0.0f;
     }
     float* fitg = a.fit + td.fit_off;
     float* Xg = a.X + td.x_off;
@@ -1311,13 +1401,16 @@ __device__ __forceinline__ void epoch_body(const EpochArgs& a, float* smem, cons
     const Rng rng{a.p.seed_lo, a.p.seed_hi, (uint32_t)task};
     const int lane = tid & 63, col = lane & 31, h = lane >> 5, wave = tid >> 6;
 
-    const int nz = L.fit - smem;  // X, Q, o, tab
-    for (int e = tid; e < nz; e += kThreads) smem[e] = 0.0f;
-    __syncthreads();
-    if constexpr (!kQGlobal<KB>) stage_rows<RS, HS>(L.Q, a.Q + td.q_off, g.D, g.D, tid);
-    for (int d = tid; d < g.D; d += kThreads) {
-        L.o[(d & 1) * HS + (d >> 1)] = a.shift[td.v_off + d];
-        L.tab[d] = a.tab[td.v_off + d];
+    if (a.init) {
+        for (int e = tid; e < g.popP * RS; e += kThreads) L.X[e] = 0.0f;
+        __syncthreads();
+    } else {
+        stage_rows<RS, HS, kThreads, 4>(L.X, a.X + td.x_off, g.pop, g.pop, g.D, KB, tid);
+    }
+    if constexpr (!kQGlobal<KB>) stage_rows<RS, HS, kThreads, 4>(L.Q, a.Q + td.q_off, g.D, 32 * NT, g.D, KB, tid);
+    for (int d = tid; d < 32 * NT; d += kThreads) {
+        if (d < 2 * HS) L.o[(d & 1) * HS + (d >> 1)] = d < g.D ? a.shift[td.v_off + d] : 0.0f;
+        L.tab[d] = d < g.D ? a.tab[td.v_off + d] : 0.0f;
     }
     if (a.init) {
         const float lo = td.lo, rng_ = td.hi - td.lo;
@@ -1336,7 +1429,6 @@ __device__ __forceinline__ void epoch_body(const EpochArgs& a, float* smem, cons
             if (i < g.pop && h == 0) L.fit[i] = f;
         }
     } else {
-        stage_rows<RS, HS>(L.X, a.X + td.x_off, g.pop, g.D, tid);
         for (int i = tid; i < g.pop; i += kThreads) L.fit[i] = a.fit[td.fit_off + i];
     }
     __syncthreads();
@@ -1359,22 +1451,20 @@ __device__ __forceinline__ void epoch_body(const EpochArgs& a, float* smem, cons
             island_migration<KB>(a, g, L, tid);
     }
 
-    float* Xg = a.X + td.x_off;
-    for (int e = tid; e < g.pop * g.D; e += kThreads) {
-        const int i = e / g.D, d = e - i * g.D;
-        Xg[e] = L.X[i * RS + (d & 1) * HS + (d >> 1)];
+    // ranked before anything is stored: a barrier waits for the stores
+    if (epub) {
+        rank_islands(L, g.pop, g.pop, tid);
+        __syncthreads();
     }
+    unstage_rows<HS, kThreads, 4>(a.X + td.x_off, L.X, [](int i) { return i * RS; }, g.pop, g.D, tid);
     for (int i = tid; i < g.pop; i += kThreads) a.fit[td.fit_off + i] = L.fit[i];
     if (epub) {
-        __syncthreads();
-        rank_islands(L, g.pop, g.pop, tid);
         if constexpr (PERSIST) {
             __shared__ int s_pub;
             if (tid == 0) s_pub = (pe == 0 || persist_wait(pa->reads + pe - 1, a.n_tasks, *pa)) ? 1 : 0;
             __syncthreads();
             if (!s_pub) return;  // the error flag is set: the launch drains
         }
-        __syncthreads();
         const int k = a.p.transfer_count;
         float* mb = a.mailbox + (int64_t)((eg1 / TI) & 1) * a.mailbox_stride + td.mb_off;
         for (int e = tid; e < k * g.D; e += kThreads) {
@@ -1813,8 +1903,9 @@ __device__ __forceinline__ void wide_gather(const Geo& g, const Lds& L, const Wi
     __syncthreads();
 }
 
-// Inter-task transfer for wide tasks: candidates streamed into the k-loop and
-// staged in T (row j for candidate j), accepted ones copied to their target row.
+// Inter-task transfer for wide tasks: the candidates are formed in T (row j for candidate j), a
+// thread per block of four genes of a half, evaluated, and the accepted ones copied to their
+// target rows.
 template <int NT, int FUNC>
 __device__ __forceinline__ void wide_transfer_in(const EpochArgs& a, const TaskDev& td, const Geo& g, const Lds& L,
                                                  float* T, const Rng& rng, int tid, int nsb) {
@@ -1822,62 +1913,62 @@ __device__ __forceinline__ void wide_transfer_in(const EpochArgs& a, const TaskD
     constexpr int RS = S::RS, HS = S::HS;
     const int k = a.p.transfer_count, TI = a.p.transfer_interval, g0 = a.g0 - td.gen_base;
     const int wave = tid >> 6, lane = tid & 63, col = lane & 31, h = lane >> 5;
-    rank_islands<kWideThreads>(L, g.pop, g.pop, tid);
-    __syncthreads();
     const uint32_t wd = rng.word((uint32_t)g0, P_MIG, 0u, 0u, 0u);
     const int dn = pick_donor(a, (int)rng.task, wd);
     const TaskDev dd = a.tasks[dn];
     const float* mb = a.mailbox + (int64_t)((a.g0 / TI) & 1) * a.mailbox_stride + dd.mb_off;
     const bool same_box = (dd.lo == td.lo && dd.hi == td.hi);
     const float rng_s = td.hi - td.lo, rng_d = dd.hi - dd.lo;
-    const float* ql = L.Q + 4 * (32 * h + col);
-    const float* orow = L.o + h * HS;
-    const int ntc = (k + 31) / 32;
-    for (int ct = wave; ct < ntc; ct += kWideThreads / 64) {
-        const int j = ct * 32 + col;
-        const bool valid = j < k;
-        const int je = valid ? j : 0;
-        const float* src = L.X + (int64_t)L.ord[je] * RS + h * HS;
-        float* crow = T + (int64_t)j * RS + h * HS;
-        f16v acc[NT];
-        zero_acc<NT>(acc);
-        for (int sb = 0; sb < nsb; ++sb) {
-            const float4 v4 = lds4(src + 4 * sb);
-            float c[4] = {v4.x, v4.y, v4.z, v4.w};
+    rank_islands<kWideThreads>(L, g.pop, g.pop, tid);
+    __syncthreads();
+    const int nu = 2 * nsb;  // blocks of a row
+    for (int e = tid; e < k * nu; e += kWideThreads) {
+        const int j = e / nu, u = e - j * nu, hh = u >= nsb ? 1 : 0, sb = u - (hh ? nsb : 0);
+        const float* mrow = mb + (int64_t)j * dd.dim;
+        float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int s = 4 * sb + e, d = 2 * s + h;
-                if (d < g.D && d < dd.dim) {
-                    bool take = true;
-                    if (a.p.transfer_cr > 0.0f) {
-                        const uint32_t wu = rng.word((uint32_t)g0, P_XFER, (uint32_t)je, (uint32_t)h, (uint32_t)s);
-                        take = uniform01(wu) > a.p.transfer_cr;
-                    }
-                    if (take) {
-                        const float v = mb[(int64_t)je * dd.dim + d];
-                        if (same_box) c[e] = v;
-                        else {
-                            const float t1 = v - dd.lo;
-                            const float t2 = t1 / rng_d;
-                            const float t3 = t2 * rng_s;
-                            c[e] = td.lo + t3;
-                        }
-                    }
+        for (int q = 0; q < 4; ++q) {
+            const int d = 2 * (4 * sb + q) + hh;
+            v[q] = mrow[d < dd.dim ? d : 0];
+        }
+        const float4 c4 = lds4(L.X + (int64_t)L.ord[j] * RS + hh * HS + 4 * sb);
+        float c[4] = {c4.x, c4.y, c4.z, c4.w};
+        U4 ub{0u, 0u, 0u, 0u};
+        if (a.p.transfer_cr > 0.0f)
+            ub = rng.block((uint32_t)g0, P_XFER, (uint32_t)j, (uint32_t)hh, (uint32_t)sb);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int d = 2 * (4 * sb + q) + hh;
+            const bool take = !(a.p.transfer_cr > 0.0f) || uniform01(pick(ub, (uint32_t)q)) > a.p.transfer_cr;
+            if (d < g.D && d < dd.dim && take) {
+                if (same_box) c[q] = v[q];
+                else {
+                    const float t1 = v[q] - dd.lo;
+                    const float t2 = t1 / rng_d;
+                    const float t3 = t2 * rng_s;
+                    c[q] = td.lo + t3;
                 }
             }
-            const float4 c4 = make_float4(c[0], c[1], c[2], c[3]);
-            *reinterpret_cast<float4*>(crow + 4 * sb) = c4;
-            mfma_block<NT>(acc, ql, sub4(c4, lds4(orow + 4 * sb)), sb);
         }
-        const float f = objective<NT, FUNC, true>(acc, g.D, L.tab, h);
-        if (valid) {
+        *reinterpret_cast<float4*>(T + (int64_t)j * RS + hh * HS + 4 * sb) = make_float4(c[0], c[1], c[2], c[3]);
+    }
+    __syncthreads();
+    const int ntc = (k + 31) / 32;
+    for (int ct = wave; ct < ntc; ct += kWideThreads / 64) {
+        const int j = ct * 32 + col, je = j < k ? j : 0;
+        const float f = wide_eval_row<NT, FUNC>(T + (int64_t)je * RS + h * HS, g, L, col, h, nsb);
+        if (j < k && h == 0) {
             const int tgt = L.ord[g.pop - k + j];
-            if (f < L.fit[tgt]) {
-                float* dst = L.X + (int64_t)tgt * RS + h * HS;
-                for (int sb = 0; sb < nsb; ++sb) *reinterpret_cast<float4*>(dst + 4 * sb) = lds4(crow + 4 * sb);
-                if (h == 0) L.fit[tgt] = f;
-            }
+            const bool acc = f < L.fit[tgt];
+            if (acc) L.fit[tgt] = f;
+            L.aux[j] = acc ? tgt : -1;
         }
+    }
+    __syncthreads();
+    for (int e = tid; e < k * nu; e += kWideThreads) {
+        const int j = e / nu, u = e - j * nu, c = u >= nsb ? HS + 4 * (u - nsb) : 4 * u;
+        const int tgt = L.aux[j];
+        if (tgt >= 0) *reinterpret_cast<float4*>(L.X + (int64_t)tgt * RS + c) = lds4(T + (int64_t)j * RS + c);
     }
     __syncthreads();
 }
@@ -1948,12 +2039,11 @@ __device__ __forceinline__ void wide_body(const EpochArgs& a, float* smem, const
         L.o[(d & 1) * HS + (d >> 1)] = a.shift[td.v_off + d];
         L.tab[d] = a.tab[td.v_off + d];
     }
-    // rows in the padded layout, zero past the dimension
-    const float* Xg = a.X + td.x_off;
-    const float lo = td.lo, rng_ = td.hi - td.lo;
-    const int nx = g.popP * RS;
+    // rows in the padded layout, zero past the dimension up to the last octet of slots that is read
+    const int nblk = 2 * ((g.Dh + 7) >> 3);
     if (a.init) {
-        for (int e = tid; e < nx; e += WT) {
+        const float lo = td.lo, rng_ = td.hi - td.lo;
+        for (int e = tid; e < g.popP * RS; e += WT) {
             const int i = e / RS, c = e - i * RS;
             const int d = (c < HS) ? 2 * c : 2 * (c - HS) + 1;
             float v = 0.0f;
@@ -1965,23 +2055,7 @@ __device__ __forceinline__ void wide_body(const EpochArgs& a, float* smem, const
             L.X[e] = v;
         }
     } else {
-        for (int e0 = tid; e0 < nx; e0 += 8 * WT) {  // eight loads in flight per thread
-            float v[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int e = e0 + k * WT;
-                const int i = e / RS, c = e - i * RS;
-                const int d = (c < HS) ? 2 * c : 2 * (c - HS) + 1;
-                const bool in = e < nx && i < g.pop && c < 2 * HS && d < g.D;
-                const float xv = Xg[in ? (int64_t)i * g.D + d : 0];
-                v[k] = in ? xv : 0.0f;
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int e = e0 + k * WT;
-                if (e < nx) L.X[e] = v[k];
-            }
-        }
+        stage_rows<RS, HS, WT, 8>(L.X, a.X + td.x_off, g.pop, g.pop, g.D, nblk, tid);
     }
     if (!a.init)
         for (int i = tid; i < g.pop; i += WT) L.fit[i] = a.fit[td.fit_off + i];
@@ -2025,16 +2099,13 @@ __device__ __forceinline__ void wide_body(const EpochArgs& a, float* smem, const
         }
     }
 
-    float* Xo = a.X + td.x_off;
-    for (int e = tid; e < g.pop * g.D; e += WT) {
-        const int i = e / g.D, d = e - i * g.D;
-        Xo[e] = L.X[W.off[i] + (d & 1) * HS + (d >> 1)];
-    }
-    for (int i = tid; i < g.pop; i += WT) a.fit[td.fit_off + i] = L.fit[i];
     if (a.publish) {
-        __syncthreads();
         rank_islands<WT>(L, g.pop, g.pop, tid);
         __syncthreads();
+    }
+    unstage_rows<HS, WT, 8>(a.X + td.x_off, L.X, [&](int i) { return W.off[i]; }, g.pop, g.D, tid);
+    for (int i = tid; i < g.pop; i += WT) a.fit[td.fit_off + i] = L.fit[i];
+    if (a.publish) {
         const int k = a.p.transfer_count;
         float* mb = a.mailbox + (int64_t)((a.g1 / TI) & 1) * a.mailbox_stride + td.mb_off;
         for (int e = tid; e < k * g.D; e += WT) {
