@@ -825,23 +825,38 @@ __device__ __forceinline__ void generation_step(const EpochArgs& a, const TaskDe
     __syncthreads();
 }
 
-// Cross-island resampling (reference SharedToGlobal + SelectFromBlocks).
+// Cross-island resampling (reference SharedToGlobal + SelectFromBlocks).  The shuffles' draws
+// and their remainders are formed by all threads, so the serial part of a shuffle is its swaps.
 template <int KB, int NTHR = kThreads>
 __device__ __forceinline__ void island_exchange(const EpochArgs& a, const Geo& g, const Lds& L, float* scr,
                                                 const Rng& rng, int gen, int tid) {
     constexpr int RS = Shape<KB>::RS;
-    const int n = a.p.n_islands, m = g.m;
+    const int n = a.p.n_islands, m = g.m, mb = (m + 3) >> 2;
+    int* draw = reinterpret_cast<int*>(L.ftmp);
+    for (int e = tid; e < n * mb; e += NTHR) {
+        const int q = e / mb, b = e - q * mb;
+        const U4 w = rng.block((uint32_t)gen, P_ISLX, (uint32_t)q, 0u, (uint32_t)b);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int k = m - 1 - (4 * b + c);
+            if (k >= 0) draw[q * m + k] = (int)(pick(w, (uint32_t)c) % (uint32_t)(k + 1));
+        }
+    }
+    for (int i = tid; i < g.pop; i += NTHR) L.aux[i] = i % m;
+    __syncthreads();
     for (int q = tid; q < n; q += NTHR) {
         int* arr = L.aux + q * m;
-        for (int p = 0; p < m; ++p) arr[p] = p;
         for (int k = m - 1; k >= 0; --k) {
-            const uint32_t w = rng.word((uint32_t)gen, P_ISLX, (uint32_t)q, 0u, (uint32_t)(m - 1 - k));
-            const int t = (int)(w % (uint32_t)(k + 1));
+            const int t = draw[q * m + k];
             const int tmp = arr[k];
             arr[k] = arr[t];
             arr[t] = tmp;
         }
-        for (int p = 0; p < m; ++p) L.ord[q * m + arr[p]] = p;  // inverse permutation
+    }
+    __syncthreads();
+    for (int i = tid; i < g.pop; i += NTHR) {  // inverse permutation
+        const int q = i / m;
+        L.ord[q * m + L.aux[i]] = i - q * m;
     }
     __syncthreads();
     // one island offset per slot k, shared by every island (the reference's
@@ -854,13 +869,36 @@ __device__ __forceinline__ void island_exchange(const EpochArgs& a, const Geo& g
         L.aux[i] = src * m + L.ord[src * m + k];
     }
     __syncthreads();
-    for (int e = tid; e < g.pop * RS; e += NTHR) {
-        const int row = e / RS, c = e - row * RS;
-        scr[e] = L.X[L.aux[row] * RS + c];
-    }
     for (int i = tid; i < g.pop; i += NTHR) L.ftmp[i] = L.fit[L.aux[i]];
-    __syncthreads();
-    for (int e = tid; e < g.pop * RS; e += NTHR) L.X[e] = scr[e];
+    if constexpr (NTHR == kThreads) {
+        // rows in LDS: permuted through registers, as many columns at a time as eight 16-byte
+        // blocks a thread hold of every row
+        constexpr int B = 8;
+        const int cols = B * NTHR / g.pop;
+        for (int c0 = 0; c0 < RS / 4; c0 += cols) {
+            const int nc = RS / 4 - c0 < cols ? RS / 4 - c0 : cols, total = g.pop * nc;
+            float4 v[B];
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                const int e = tid + b * NTHR, row = e / nc, c = c0 + e - row * nc;
+                if (e < total) v[b] = lds4(L.X + L.aux[row] * RS + 4 * c);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                const int e = tid + b * NTHR, row = e / nc, c = c0 + e - row * nc;
+                if (e < total) *reinterpret_cast<float4*>(L.X + row * RS + 4 * c) = v[b];
+            }
+        }
+    } else {
+        for (int e = tid; e < g.pop * (RS / 4); e += NTHR) {
+            const int row = e / (RS / 4), c = 4 * (e - row * (RS / 4));
+            *reinterpret_cast<float4*>(scr + 4 * e) = lds4(L.X + L.aux[row] * RS + c);
+        }
+        __syncthreads();
+        for (int e = tid; e < g.pop * (RS / 4); e += NTHR)
+            *reinterpret_cast<float4*>(L.X + 4 * e) = lds4(scr + 4 * e);
+    }
     for (int i = tid; i < g.pop; i += NTHR) L.fit[i] = L.ftmp[i];
     __syncthreads();
 }

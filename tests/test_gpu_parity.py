@@ -515,3 +515,24 @@ def test_elites_on_both_sides_of_the_pinned_size(n_tasks):
             order = np.argsort(fp, kind="stable")[:k]
             assert np.array_equal(f[t], fp[order]), f"task {t} k {k}"
             assert np.array_equal(x[t][:, :67], xp[order]), f"task {t} k {k}"
+
+
+@pytest.mark.parametrize("algo, pop, n_islands", [(emtf.DE_RAND_1_BIN, 6, 2), (emtf.DE_RAND_1_BIN, 36, 4),
+                                                  (emtf.DE_RAND_1_BIN, 252, 12), (emtf.DE_RAND_1_BIN, 512, 8),
+                                                  (emtf.GA_SBX_PM, 12, 2), (emtf.GA_SBX_PM, 36, 6),
+                                                  (emtf.GA_SBX_PM, 252, 14), (emtf.GA_SBX_PM, 512, 8)])
+def test_rows_in_and_out_of_an_epoch(oracle_mod, algo, pop, n_islands):
+    """Every remainder of a row's last block of eight genes, in the LDS and the wide kernel;
+    islands whose exchange takes one pass over the columns or several and whose sizes leave
+    remainders of a draw's four words; candidates from other boxes, gene by gene."""
+    dims = [1, 2, 3, 4, 5, 6, 7, 8, 9, 15, 31, 50, 58, 70, 101] + ([129, 130, 131, 132, 133, 134, 135, 136] if pop < 512 else [])
+    tasks = tg.benchmark_tasks(len(dims), 0, pop, rotate=True, seed=59, dims=dims)
+    for t in tasks[1::3]:
+        t["lo"], t["hi"] = -50.0, 70.0
+    params = dict(seed=9, algo=algo, n_islands=n_islands, exchange_interval=2, migrate_interval=3, migrate_count=1,
+                  transfer_interval=3, transfer_count=3, transfer_cr=0.4)
+    gpu, orc = _pair(tasks, oracle_mod, tune=1, **params)
+    for step in (3, 4):
+        gpu.run(step)
+        orc.run(step)
+        _compare(gpu, orc, f"rows pop {pop} islands {n_islands} gen {orc.generation}")
