@@ -788,6 +788,7 @@ __device__ __forceinline__ void generation_step(const EpochArgs& a, const TaskDe
     float fchild = 0.0f;
     int i_keep = -1;
     bool acc_keep = false;
+    unsigned taken = 0u;  // multi: the wave's tiles whose trial the lane took
     for (int it = wave; it < g.ntiles; it += kThreads / 64) {
         const int i = it * 32 + col;
         const bool valid = i < g.pop;
@@ -796,7 +797,8 @@ __device__ __forceinline__ void generation_step(const EpochArgs& a, const TaskDe
         const bool accept = valid && (L.fit[i] >= f);
         if (multi) {
             if (accept) store_half_row<KB>(a.scratch + td.scr_off + (int64_t)i * S::RS + h * S::HS, tr);
-            if (valid && h == 0) { L.aux[i] = accept ? 1 : 0; L.ftmp[i] = f; }
+            if (accept && h == 0) L.ftmp[i] = f;
+            taken |= accept ? 1u << (it / (kThreads / 64)) : 0u;
         } else {
             i_keep = i;
             acc_keep = accept;
@@ -810,17 +812,14 @@ __device__ __forceinline__ void generation_step(const EpochArgs& a, const TaskDe
             if (h == 0) L.fit[i_keep] = fchild;
         }
     } else {
-        const float* src = a.scratch + td.scr_off;
-        for (int e = tid; e < g.pop * (2 * KB); e += kThreads) {
-            const int row = e / (2 * KB), blk = e - row * (2 * KB);
-            if (L.aux[row]) {
-                const int c = (blk < KB) ? 4 * blk : S::HS + 4 * (blk - KB);
-                *reinterpret_cast<float4*>(L.X + row * S::RS + c) =
-                    *reinterpret_cast<const float4*>(src + (int64_t)row * S::RS + c);
-            }
+        // each lane fetches the half rows that it left in scratch memory
+        for (int it = wave; it < g.ntiles; it += kThreads / 64) {
+            if (!((taken >> (it / (kThreads / 64))) & 1u)) continue;
+            const int i = it * 32 + col;
+            load_half_row<KB>(tr, a.scratch + td.scr_off + (int64_t)i * S::RS + h * S::HS);
+            store_half_row<KB>(L.X + i * S::RS + h * S::HS, tr);
+            if (h == 0) L.fit[i] = L.ftmp[i];
         }
-        for (int i = tid; i < g.pop; i += kThreads)
-            if (L.aux[i]) L.fit[i] = L.ftmp[i];
     }
     __syncthreads();
 }
