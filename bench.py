@@ -79,7 +79,7 @@ def parse():
     ap.add_argument("--one-call", action="store_true",
                     help="run the timed steps as one emtf_run call (the persistent schedule's single launch)")
     ap.add_argument("--schedule", default="auto", choices=["auto", "epochs", "persistent"],
-                    help="auto: epochs replayed from a captured hipGraph; epochs: launched directly; "
+                    help="auto: epochs of several launch units replayed from a captured hipGraph; epochs: launched directly; "
                          "persistent: one launch per run, epochs ordered on the device")
     return ap.parse_args()
 
@@ -522,7 +522,8 @@ def main():
                      "avg_launch_ms": gpu_ms / a.steps},
         "cpu_baseline": cpu,
         "time_to_1e-6": study,
-        "launch": {"auto": "epochs replayed from a captured hipGraph", "epochs": "epochs launched directly",
+        "launch": {"auto": "epochs launched directly (one launch unit) or replayed from a captured hipGraph (several)",
+                   "epochs": "epochs launched directly",
                    "persistent": "persistent schedule, epochs ordered on the device"}[a.schedule]
                   + (f"; the {a.steps} steps as one run call" if a.one_call else ""),
         "wall_s": wall,
