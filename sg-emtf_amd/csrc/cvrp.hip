@@ -33,7 +33,8 @@
 namespace emtf {
 
 constexpr uint32_t P_CV_INIT = 16, P_CV_GEN = 17;
-constexpr int kCvThreads = 512;  // eight waves: two workgroups of n = 200 share a CU
+constexpr int kCvThreads = 512;  // eight waves: two workgroups of n = 200 share a CU; twice that
+                                 // where a CU has one instance at most (emtf_cvrp_launch)
 constexpr int kCvBatch = 64;     // individuals per pass
 constexpr int kSlots = 16;       // window positions in registers; longer windows read the rest from LDS
 
@@ -359,9 +360,9 @@ __device__ __forceinline__ int split_min(RowT* row, int n, int woff, int sub) {
     return 0;  // not reached: n - j0 < 16
 }
 
-template <typename RowT>
+template <int NTHR, typename RowT>
 __device__ __forceinline__ void rank_cost(const CvLds<RowT>& L, int pop, int m, int tid) {
-    for (int i = tid; i < pop; i += kCvThreads) {
+    for (int i = tid; i < pop; i += NTHR) {
         const int q = i / m, base = q * m, il = i - base;
         const int32_t fi = L.cost[i];
         int r = 0;
@@ -373,8 +374,8 @@ __device__ __forceinline__ void rank_cost(const CvLds<RowT>& L, int pop, int m, 
     }
 }
 
-template <typename RowT>
-__global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4))) void cvrp_epoch_kernel(
+template <typename RowT, int NTHR>
+__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4))) void cvrp_epoch_kernel(
     CvrpArgs a, const int* __restrict__ order) {
     extern __shared__ __align__(16) uint8_t cv_smem[];
     const int inst = order[blockIdx.x];
@@ -400,20 +401,20 @@ __global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4)))
     const Rng rng{a.seed_lo, a.seed_hi, (uint32_t)inst};
     const int m = pop / (a.n_islands > 0 ? a.n_islands : 1);
 
-    for (int e = tid; e < S; e += kCvThreads) {
+    for (int e = tid; e < S; e += NTHR) {
         const uint32_t c = a.xy[cd.xy_off + e];
         L.node[e] = make_uint2(c, (uint32_t)nint_xy(0u, c) | ((uint32_t)a.dem[cd.dem_off + e] << 8));
     }
-    for (int i = tid; i < popP; i += kCvThreads) L.cur[i] = 0;
+    for (int i = tid; i < popP; i += NTHR) L.cur[i] = 0;
     uint8_t* tg = a.tours + cd.tour_off;
     if (!a.init) {
-        for (int e = tid; e < pop * n; e += kCvThreads) {
+        for (int e = tid; e < pop * n; e += NTHR) {
             const int i = e / n, k = e - i * n;
             L.T[i * NP + k] = tg[e];
         }
-        for (int i = tid; i < pop; i += kCvThreads) L.cost[i] = a.cost[cd.cost_off + i];
+        for (int i = tid; i < pop; i += NTHR) L.cost[i] = a.cost[cd.cost_off + i];
     } else {
-        for (int i = tid; i < pop; i += kCvThreads) {
+        for (int i = tid; i < pop; i += NTHR) {
             uint8_t* tour = L.T + i * NP;
             for (int k = 0; k < n; ++k) tour[k] = (uint8_t)(k + 1);
             U4 blk{0u, 0u, 0u, 0u};
@@ -450,7 +451,7 @@ __global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4)))
     if (a.init) {
         for (int i0 = 0; i0 < pop; i0 += kCvBatch) {
             const int cnt = pop - i0 < kCvBatch ? pop - i0 : kCvBatch;
-            for (int q = wave; q < cnt; q += kCvThreads / 64) {
+            for (int q = wave; q < cnt; q += NTHR / 64) {
                 const uint8_t* const t[1] = {L.T + (i0 + q) * NP};
                 RowT* const row[1] = {L.G + q * GW};
                 int32_t* const info[1] = {L.info + q};
@@ -467,7 +468,7 @@ __global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4)))
         for (int i0 = 0; i0 < pop; i0 += kCvBatch) {
             const int cnt = pop - i0 < kCvBatch ? pop - i0 : kCvBatch;
             // lane l draws for the wave's l-th individual of the pass (row wave + 8 l)
-            const int ql = wave + (kCvThreads / 64) * (lane & 7);
+            const int ql = wave + (NTHR / 64) * (lane & 7);
             const int i = i0 + (ql < cnt ? ql : 0);
             const int il = i % m, base = i - il;
             const U4 b0 = rng.block((uint32_t)gen, P_CV_GEN, (uint32_t)i, 0u, 0u);
@@ -492,8 +493,8 @@ __global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4)))
                 int32_t* info[NI];
 #pragma unroll
                 for (int e = 0; e < NI; ++e) {
-                    const int le = wave + (kCvThreads / 64) * (l + e) < cnt ? l + e : l;
-                    const int q = wave + (kCvThreads / 64) * le;
+                    const int le = wave + (NTHR / 64) * (l + e) < cnt ? l + e : l;
+                    const int q = wave + (NTHR / 64) * le;
                     const uint32_t v = (uint32_t)__builtin_amdgcn_readlane(cuts, le);
                     const uint32_t w = (uint32_t)__builtin_amdgcn_readlane(rest, le);
                     const int self = (w >> 12) & 1, mt = (w >> 10) & 3;
@@ -517,7 +518,7 @@ __global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4)))
                 split_data<NC, NI>(t, row, info, L.node, n, cap, lane);
             };
             using std::integral_constant;
-            for (int l = 0; wave + (kCvThreads / 64) * l < cnt; l += n <= 128 ? 2 : 1) {
+            for (int l = 0; wave + (NTHR / 64) * l < cnt; l += n <= 128 ? 2 : 1) {
                 if (n <= 64) breed(integral_constant<int, 1>{}, integral_constant<int, 2>{}, l);
                 else if (n <= 128) breed(integral_constant<int, 2>{}, integral_constant<int, 2>{}, l);
                 else if (n <= 192) breed(integral_constant<int, 3>{}, integral_constant<int, 1>{}, l);
@@ -528,22 +529,22 @@ __global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4)))
             __syncthreads();
         }
         // accepted children become the individuals once every child of the generation is made
-        for (int i = tid; i < pop; i += kCvThreads) {
+        for (int i = tid; i < pop; i += NTHR) {
             const int c = L.cur[i];
             L.cur[i] = (c ^ (c >> 1)) & 1;
         }
         __syncthreads();
         const int nis = a.n_islands, kk = a.migrate_count;
         if (nis > 1 && a.migrate_interval > 0 && kk > 0 && gen % a.migrate_interval == 0) {
-            rank_cost(L, pop, m, tid);
+            rank_cost<NTHR>(L, pop, m, tid);
             __syncthreads();
-            for (int e = tid; e < nis * kk; e += kCvThreads) {
+            for (int e = tid; e < nis * kk; e += NTHR) {
                 const int q = e / kk, j = e - q * kk, pd = (q + 1) % nis;
                 const int src = L.ord[q * m + j], dst = L.ord[pd * m + m - kk + j];
                 L.aux[e] = (L.cost[src] < L.cost[dst]) ? 1 : 0;
             }
             __syncthreads();
-            for (int e = tid; e < nis * kk * (NP / 4); e += kCvThreads) {
+            for (int e = tid; e < nis * kk * (NP / 4); e += NTHR) {
                 const int pr = e / (NP / 4), w = e - pr * (NP / 4);
                 if (L.aux[pr]) {
                     const int q = pr / kk, j = pr - q * kk, pd = (q + 1) % nis;
@@ -552,7 +553,7 @@ __global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4)))
                         reinterpret_cast<const uint32_t*>(L.T + L.cur[src] * TN + src * NP)[w];
                 }
             }
-            for (int e = tid; e < nis * kk; e += kCvThreads) {
+            for (int e = tid; e < nis * kk; e += NTHR) {
                 if (L.aux[e]) {
                     const int q = e / kk, j = e - q * kk, pd = (q + 1) % nis;
                     const int src = L.ord[q * m + j], dst = L.ord[pd * m + m - kk + j];
@@ -562,11 +563,11 @@ __global__ __launch_bounds__(kCvThreads) __attribute__((amdgpu_waves_per_eu(4)))
             __syncthreads();
         }
     }
-    for (int e = tid; e < pop * n; e += kCvThreads) {
+    for (int e = tid; e < pop * n; e += NTHR) {
         const int i = e / n, k = e - i * n;
         tg[e] = L.T[L.cur[i] * TN + i * NP + k];
     }
-    for (int i = tid; i < pop; i += kCvThreads) a.cost[cd.cost_off + i] = L.cost[i];
+    for (int i = tid; i < pop; i += NTHR) a.cost[cd.cost_off + i] = L.cost[i];
 }
 
 // Best individual of every instance (the first of the smallest cost), one wave each: its cost
@@ -617,23 +618,29 @@ extern "C" int emtf_cvrp_lds_bytes(int n, int popP, int entry_bytes) {
     return emtf::cvrp_lds_bytes(n, popP, entry_bytes);
 }
 
+template <typename RowT, int NTHR>
+static hipError_t launch_epoch(const emtf::CvrpArgs& a, const int* order, int n, int lds_bytes, hipStream_t stream) {
+    static bool lds_ok = false;
+    auto k = &emtf::cvrp_epoch_kernel<RowT, NTHR>;
+    if (!lds_ok) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return e;
+        lds_ok = true;
+    }
+    hipLaunchKernelGGL(k, dim3(n), dim3(NTHR), lds_bytes, stream, a, order);
+    return hipGetLastError();
+}
+
 // entry_bytes 2: W + woff in 16 bits (the host checks that every instance's W + woff range
-// fits); else W in 32 bits.
+// fits); else W in 32 bits.  Sixteen waves an instance up to one instance a CU (the registers of
+// sixteen waves fill it), eight beyond.  100 generations, 50 to 200 customers, pop 128: 16 / 256
+// instances 6.21 / 6.33 ms with eight waves, 5.07 / 5.21 with sixteen; 512 instances 6.55 and 7.20.
 extern "C" int emtf_cvrp_launch(const emtf::CvrpArgs* args, const int* order, int n_inst, int lds_bytes, int entry_bytes,
                                 hipStream_t stream) {
-    static bool lds_ok[2] = {false, false};
-    const int w = entry_bytes == 2 ? 0 : 1;
-    const void* k = w == 0 ? reinterpret_cast<const void*>(&emtf::cvrp_epoch_kernel<uint16_t>)
-                           : reinterpret_cast<const void*>(&emtf::cvrp_epoch_kernel<uint32_t>);
-    if (!lds_ok[w]) {
-        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        if (e != hipSuccess) return (int)e;
-        lds_ok[w] = true;
-    }
-    const dim3 block(emtf::kCvThreads);
-    if (w == 0)
-        hipLaunchKernelGGL(emtf::cvrp_epoch_kernel<uint16_t>, dim3(n_inst), block, lds_bytes, stream, *args, order);
-    else
-        hipLaunchKernelGGL(emtf::cvrp_epoch_kernel<uint32_t>, dim3(n_inst), block, lds_bytes, stream, *args, order);
-    return (int)hipGetLastError();
+    constexpr int kCus = 256;
+    const bool wide = args->n_inst <= kCus;
+    auto* const fn = entry_bytes == 2 ? (wide ? &launch_epoch<uint16_t, 2 * emtf::kCvThreads> : &launch_epoch<uint16_t, emtf::kCvThreads>)
+                                      : (wide ? &launch_epoch<uint32_t, 2 * emtf::kCvThreads> : &launch_epoch<uint32_t, emtf::kCvThreads>);
+    return (int)fn(*args, order, n_inst, lds_bytes, stream);
 }

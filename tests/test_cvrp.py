@@ -232,3 +232,29 @@ def test_gpu_cvrp_chunk_edges(oracle_mod, pop, n_islands):
         assert np.array_equal(tg, to), i
         b = int(np.argmin(co))
         assert cost[i] == co[b] and np.array_equal(tour[i, :inst[i]["n"]], to[b]) and not tour[i, inst[i]["n"]:].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_inst", [256, 257])
+def test_gpu_cvrp_waves_per_instance(oracle_mod, n_inst):
+    """On both sides of one instance per compute unit (sixteen and eight waves an instance):
+    every tour and cost bit-exact with the oracle, tours of one to four chunks."""
+    from emtf.cvrp import CvrpEngine
+    rng = np.random.default_rng(n_inst)
+    inst = []
+    for k in range(n_inst):
+        n = (3, 64, 65, 129, 200)[k % 5]
+        xy = np.vstack([[50, 50], rng.integers(0, 101, (n, 2))]).astype(np.int32)
+        dem = np.concatenate([[0], rng.integers(1, 11, n)]).astype(np.int32)
+        inst.append(dict(n=n, capacity=(12, 50, 62)[k % 3], pop=70, xy=xy, demand=dem))
+    params = dict(p_swap=0.3, p_2opt=0.3, n_islands=2, migrate_interval=2, migrate_count=1, seed=7)
+    print("case: cvrp waves, instances", n_inst, flush=True)
+    gpu = CvrpEngine(inst, **params)
+    orc = oracle_mod.CvrpEngine(inst, **params)
+    gpu.run(4)
+    orc.run(4)
+    for i in range(n_inst):
+        tg, cg = gpu.population(i)
+        to, co = orc.population(i)
+        assert np.array_equal(cg, co), i
+        assert np.array_equal(tg, to), i
