@@ -191,6 +191,12 @@ int emtf_cvrp_create(const emtf_cvrp_instance* in, int32_t n_inst, const emtf_cv
         if (b > kMaxLds || need > kMaxLds) { cv_free(h); return cfail(EMTF_E_UNSUPPORTED, "instance exceeds LDS"); }
         occ[t] = std::min(4, kMaxLds / b);  // 512 threads: four workgroups fill a CU
     }
+    // a batch that is resident as a whole at the largest instance's occupancy is one launch:
+    // groups on streams that share a hardware queue run one after another (512 instances of 50
+    // to 200 customers, 100 generations: 6.5 ms beside each other, 7.8 where two shared one)
+    constexpr int kCus = 256;
+    const int least = *std::min_element(occ.begin(), occ.end());
+    if (n_inst <= least * kCus) std::fill(occ.begin(), occ.end(), least);
     std::vector<int> order(n_inst);
     for (int t = 0; t < n_inst; ++t) order[t] = t;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
